@@ -143,6 +143,15 @@ def decode_paged(q, key_pages, value_pages, block_table, *, length, seq_lens=Non
     return out
 
 
+def _split_workspace(L, device, *sizes):
+    """Workspace of its own for an MFMA prefill that cuts its key ranges over
+    several blocks (None where the chunk runs unsplit): from torch's
+    stream-ordered allocator, so that calls on different streams share
+    nothing.  ``sizes``: the arguments of alpx_prefill_split_bytes."""
+    nbytes = L.alpx_prefill_split_bytes(*sizes)
+    return _torch().empty(nbytes, dtype=_torch().uint8, device=device) if nbytes else None
+
+
 def prefill_append(q, key, value, key_cache, value_cache, *, position, scale=None, window=0,
                    out_dtype=None, gate=None):
     """Writes the chunk's rows ``key/value [T, Hkv, D]`` to rows ``position ..``
@@ -163,7 +172,9 @@ def prefill_append(q, key, value, key_cache, value_cache, *, position, scale=Non
     if nbytes == 0:
         raise ValueError("invalid prefill sizes")
     fast = (q.dtype != torch.float32 and key_dim == value_dim and key_dim in (64, 128, 256))
-    ws = None if fast else _lib.workspace(torch, q.device, nbytes)
+    ws = (_split_workspace(L, q.device, q_tokens, int(position) + q_tokens, q_heads, kv_heads,
+                           key_dim, int(position), int(window), 0)
+          if fast else _lib.workspace(torch, q.device, nbytes))
 
     def call(workspace):
         return L.alpx_prefill_append(
@@ -177,8 +188,8 @@ def prefill_append(q, key, value, key_cache, value_cache, *, position, scale=Non
 
     rc = call(ws)
     # unaligned rows or a cache of 2 GiB or more leave the MFMA kernels; the
-    # split-K path refuses a null workspace before its append
-    if rc == _lib.EINVAL and ws is None:
+    # split-K path refuses a null or small workspace before its append
+    if rc == _lib.EINVAL and fast:
         ws = _lib.workspace(torch, q.device, nbytes)
         rc = call(ws)
     _lib.check(rc)
@@ -398,9 +409,11 @@ def prefill(q, key, value, *, pos0, scale=None, window=0, kv_start=0, kv_tokens=
     nbytes = L.alpx_prefill_workspace_bytes(q_tokens, q_heads, kv_heads, value_dim, kv_tokens)
     if nbytes == 0:
         raise ValueError("invalid prefill sizes")
-    # only the split-K fallback (fp32, odd shapes) touches the workspace
+    # the split-K fallback (fp32, odd shapes) needs the workspace
     fast = (q.dtype != torch.float32 and key_dim == value_dim and key_dim in (64, 128, 256))
-    ws = None if fast else _lib.workspace(torch, q.device, nbytes)
+    ws = (_split_workspace(L, q.device, q_tokens, int(kv_tokens), q_heads, kv_heads, key_dim,
+                           int(pos0), int(window), int(kv_start))
+          if fast else _lib.workspace(torch, q.device, nbytes))
 
     def call(workspace):
         args = (None if workspace is None else workspace.data_ptr(),
@@ -415,7 +428,7 @@ def prefill(q, key, value, *, pos0, scale=None, window=0, kv_start=0, kv_tokens=
                                            gate.data_ptr(), out.data_ptr(), *args)
 
     rc = call(ws)
-    if rc == _lib.EINVAL and ws is None:  # unaligned rows fell back: retry with workspace
+    if rc == _lib.EINVAL and fast:  # unaligned rows fell back: retry with its workspace
         ws = _lib.workspace(torch, q.device, nbytes)
         rc = call(ws)
     _lib.check(rc)
@@ -774,13 +787,16 @@ def attention_layer_prefill(query_gate, key, value, q_norm, k_norm, key_cache, v
 
     # Every refusal below comes before the library's first launch, so a
     # refused form has written nothing and the next form may run.
+    split = L.alpx_prefill_split_bytes(tokens, int(position) + tokens, q_heads, kv_heads, dim,
+                                       int(position), 0, 0) if fast else 0
     if fused_query:
-        rc = call(None, _lib.workspace(torch, dev, max(tokens * pairs * 8, 1)))
+        table = (tokens * pairs * 8 + 255) // 256 * 256
+        rc = call(None, _lib.workspace(torch, dev, max(table + split, 1)))
         if not (auto and rc == _lib.EUNSUPPORTED):  # e.g. a cache of 2 GiB or more
             _lib.check(rc)
             return out
     query = torch.empty((tokens, q_heads, dim), dtype=key_cache.dtype, device=dev)
-    rc = call(query, None)
+    rc = call(query, _lib.workspace(torch, dev, split) if split else None)
     if rc == _lib.EINVAL:  # the split-K prefill (fp32, unaligned, >= 2 GiB) needs a workspace
         nbytes = L.alpx_prefill_workspace_bytes(tokens, q_heads, kv_heads, dim,
                                                 int(position) + tokens)

@@ -245,6 +245,19 @@ size_t alpx_prefill_workspace_bytes(int q_tokens, int q_heads, int kv_heads, int
                                     int kv_tokens);
 
 /*
+ * Workspace bytes with which the MFMA prefill (alpx_prefill_causal,
+ * alpx_prefill_causal_gated, alpx_prefill_append) cuts this chunk's key
+ * ranges over more blocks and merges their partial states in a second
+ * launch; 0 where it runs the chunk unsplit.  Given less (or null), it runs
+ * unsplit: the same result within rounding, slower.  The calls that share
+ * such a workspace must be ordered, so give calls on different streams one
+ * each.  alpx_attention_layer_prefill without query_out uses what follows
+ * its tokens x R x 8 bytes, rounded up to 256.
+ */
+size_t alpx_prefill_split_bytes(int q_tokens, int kv_tokens, int q_heads, int kv_heads,
+                                int head_dim, int64_t q_pos0, int window, int64_t kv_start);
+
+/*
  * Causal (optionally sliding-window) GQA prefill attention.
  * Replaces Model._attention_batch_np (model.py:1254-1272), its windowed form
  * _attention_batch_window_np (model.py:1567-1592), the device seam
@@ -261,7 +274,8 @@ size_t alpx_prefill_workspace_bytes(int q_tokens, int q_heads, int kv_heads, int
  * q_pos0 + t - window).  A row that sees no key yields zeros (the device
  * seam's convention, cuda.py:572-577).  Scale is usually 1/sqrt(key_dim).
  * fp16/bf16 with key_dim == value_dim in {64, 128, 256} and 16-byte aligned
- * rows run the MFMA flash kernel (no workspace); anything else runs the
+ * rows run the MFMA flash kernel (which needs no workspace and takes
+ * alpx_prefill_split_bytes of it where given); anything else runs the
  * split-K machinery and needs alpx_prefill_workspace_bytes of workspace.
  */
 int alpx_prefill_causal(const void* q, const void* key, const void* value, void* out,

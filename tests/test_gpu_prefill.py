@@ -150,6 +150,65 @@ def test_prefill_append_equals_append_then_prefill(gpu, override, kernel, dtype,
     assert err <= TOL[dtype], err
 
 
+@pytest.mark.parametrize("dtype,tq,prefix,hq,hkv,d,window,kv_start,form", [
+    ("bf16", 9, 1100, 32, 8, 128, 0, 0, "append"), ("f16", 77, 2011, 12, 4, 128, 0, 0, "append"),
+    ("bf16", 33, 1537, 16, 2, 256, 0, 0, "gated"), ("f16", 40, 4000, 8, 2, 64, 2100, 0, "plain"),
+    ("bf16", 1100, 0, 1, 1, 128, 0, 5, "plain"), ("bf16", 300, 1600, 6, 2, 128, 1500, 70, "gated"),
+    ("bf16", 130, 1700, 16, 2, 256, 0, 0, "layer"), ("f16", 21, 2500, 8, 2, 128, 0, 0, "layer"),
+    ("bf16", 200, 8000, 48, 8, 64, 0, 0, "append")])
+def test_prefill_split_matches_unsplit_and_oracle(gpu, ops, override, dtype, tq, prefix, hq, hkv,
+                                                  d, window, kv_start, form):
+    """Chunks whose key ranges are cut over several blocks and merged by a
+    second launch: a last piece shorter than the others, column tiles with
+    fewer pieces than the heaviest, groups that do not divide a block's
+    columns, 16-column fragments past the last column, windows, rows that see
+    no key, one piece (the two wave groups alone), through the append, the
+    gated and the attention-layer form.  Against the unsplit kernel and the
+    oracle at the dtype's bar; caches bit for bit."""
+    import torch
+    P, lib = _mod("_ops"), _mod("_lib").lib()
+    total = prefix + tq
+    assert lib.alpx_prefill_split_bytes(tq, total, hq, hkv, d, prefix + kv_start - (kv_start and 5),
+                                        window, kv_start) > 0
+    rng = np.random.default_rng(tq + prefix + d)
+    r = lambda *s: I.round_to(rng.standard_normal(s), dtype)  # noqa: E731
+    q, K, V, gate = r(tq, hq, d), r(total, hkv, d), r(total, hkv, d), r(tq, hq, d)
+    outs, caches = [], []
+    for kernel in ("auto", "single"):
+        override("prefill_kernel", kernel)
+        kc, vc = (_dev(torch, np.concatenate([x[:prefix], np.zeros_like(x[prefix:])])[:, None],
+                       dtype, gpu) for x in (K, V))
+        if form == "append":
+            out = P.prefill_append(_dev(torch, q, dtype, gpu), _dev(torch, K[prefix:], dtype, gpu),
+                                   _dev(torch, V[prefix:], dtype, gpu), kc, vc, position=prefix,
+                                   window=window, out_dtype=torch.float32)
+        elif form == "layer":
+            qg = _dev(torch, np.concatenate([q, gate], -1).reshape(tq, -1), dtype, gpu)
+            w = torch.linspace(0.5, 1.5, d, device=gpu)
+            out, _ = ops.attention_layer_prefill_(
+                qg, _dev(torch, K[prefix:].reshape(tq, -1), dtype, gpu),
+                _dev(torch, V[prefix:].reshape(tq, -1), dtype, gpu), w, w, kc, vc,
+                position=prefix, sections=(11, 11, 10, 0), frequency_base=1e7, epsilon=1e-6)
+        else:
+            # with kv_start the first rows (5 of them) may see no key
+            out = P.prefill(_dev(torch, q, dtype, gpu), _dev(torch, K, dtype, gpu),
+                            _dev(torch, V, dtype, gpu), pos0=prefix + kv_start - (kv_start and 5),
+                            window=window, kv_start=kv_start, out_dtype=torch.float32,
+                            gate=_dev(torch, gate, dtype, gpu) if form == "gated" else None)
+        torch.cuda.synchronize()
+        outs.append(out.float())
+        caches.append((kc.view(torch.int16), vc.view(torch.int16)))
+    assert torch.equal(caches[0][0], caches[1][0]) and torch.equal(caches[0][1], caches[1][1])
+    assert (outs[0] - outs[1]).abs().max().item() <= TOL[dtype]
+    if form == "layer":
+        return  # the unsplit chunk is checked against the token chain elsewhere
+    ref = A.attention_batch(q, K, V, prefix + kv_start - (kv_start and 5) + np.arange(tq),
+                            hq // hkv, 1.0 / np.sqrt(d), window=window, kv_start=kv_start)
+    if form == "gated":
+        ref = ref / (1.0 + np.exp(-gate))
+    assert np.abs(outs[0].cpu().numpy() - ref).max() <= TOL[dtype]
+
+
 def test_prefill_append_range_error_leaves_cache(gpu):
     import torch
     P = _mod("_ops")
