@@ -178,9 +178,11 @@ SplitPlan plan_split_prefill(int q_tokens, int kv_tokens, int q_heads, int kv_he
 // of pairs) 1.02.  So: pairs must form one round that fills the device,
 // and the heaviest column tile must walk at least R times the key tiles of
 // the lightest, R = 3 at head_dim 128 and 1.8 at 64 and 256.  At head_dim
-// 256 several rounds of pairs pay as well (16/2 heads, pair / single:
-// 4096 tokens at prefix 0 -- 162 / 232 us, at prefix 1024 -- 240 / 292,
-// 8192 tokens at prefix 0 -- 656 / 859).  The shared-stream kernel (one
+// 256 two full rounds of pairs do no worse (16/2 heads, pair / single:
+// 4096 tokens at prefix 0 -- 168 / 169 us, at prefix 1024 -- 236 / 240);
+// partly filled rounds do (3000 tokens at prefix 0 -- 121 / 103; 24/4
+// heads, 1536 tokens -- 76 / 47), as do three (24/4 heads, 4096 tokens --
+// 248 / 240).  The shared-stream kernel (one
 // tile stream for both tiles of a pair, no window start inside the chunk)
 // pays off at head_dim 256 with long prefixes only (2048 tokens, 16/2
 // heads, shared / pair / single, us, one box: prefix 1024 -- 86.9 / 82.7 /
@@ -207,8 +209,10 @@ PrefillKernelChoice choose_prefill(int q_tokens, int kv_tokens, int kv_heads, in
   const int64_t pairs = (int64_t)kv_heads * ((col_tiles + 1) / 2);
   const int resident = alpx::resident_blocks(pair_kernel, 512, 0);
   if (resident <= 0) return kSingleKernel;
-  const bool one_round = pairs <= resident && pairs * 10 >= (int64_t)resident * 9;
-  if (!one_round && !(key_dim == 256 && pairs > resident)) return kSingleKernel;
+  const int64_t rounds = (pairs + resident - 1) / resident;
+  const bool one_round = rounds == 1;
+  if (pairs * 10 < rounds * resident * 9 || rounds > (key_dim == 256 ? 2 : 1))
+    return kSingleKernel;
   const int first = host_tile_keys(q_tokens, kv_tokens, group, rel0, window, cols_per_block, rows, 0);
   const int last =
       host_tile_keys(q_tokens, kv_tokens, group, rel0, window, cols_per_block, rows, col_tiles - 1);

@@ -67,20 +67,32 @@ struct PrefillArgs {
 
 constexpr int kXcds = 8;  // MI355X: workgroup b is dispatched to XCD b % 8
 
-// XCD-aware work mapping.  Work items (kv head, column tile) are ordered
-// kv-head-major, heaviest column tile first, and cut into 8 contiguous
-// slices, slice x running on XCD x, so the blocks of one kv head share one
-// XCD's L2 and its K/V tiles are fetched from HBM once instead of once per
-// XCD.  Inside a slice the first half of the dispatch order takes the heavy
-// items in descending order and the second half the light items in
-// ascending order, so the two blocks that share a CU (dispatched one slice
-// pass apart) carry a heavy and a light tile.
+// XCD-aware work mapping.  The blocks of one kv head share one XCD's L2 (or
+// as few XCDs as the head count allows), so its K/V tiles are fetched from
+// HBM once instead of once per XCD.  With 1, 2 or 4 kv heads, each head has
+// 8, 4 or 2 XCDs, which take its column tiles in turn, so that every XCD
+// gets the same share of light and heavy tiles; otherwise, and where a
+// window keeps neighbouring tiles to the same keys, the work items (kv
+// head, column tile), kv-head-major and heaviest tile first, are cut into 8
+// contiguous slices, slice x on XCD x.  Inside an XCD's share the first
+// half of the dispatch order takes the heavy items in descending order and
+// the second half the light items in ascending order, so the two blocks
+// that share a CU (dispatched one pass apart) carry a heavy and a light
+// tile.  Contiguous slices / tiles in turn, us (one box, bf16): 16/2 heads of
+// 256, 2048 tokens 65 / 58, 3000 tokens 157 / 103; 32/4 heads of 128, 3000
+// tokens 122 / 98; 32/1, 4096 tokens 216 / 157; with a window of 512 rows,
+// 16/2 heads of 256, 3000 tokens 45 / 47.
 __device__ __forceinline__ bool prefill_work(const PrefillArgs& a, int& kvh, int& ctile) {
-  const int b = blockIdx.x;
-  const int j = b / kXcds;
+  const int b = blockIdx.x, x = b % kXcds, j = b / kXcds;
   const int half = (a.per_xcd + 1) / 2;
   const int rank = j < half ? j : a.per_xcd - 1 - (j - half);
-  const int item = (b % kXcds) * a.per_xcd + rank;
+  if (a.window <= 0 && a.kv_heads <= 4 && a.kv_heads != 3) {
+    const int share = kXcds / a.kv_heads;  // XCDs per head
+    kvh = x / share;
+    ctile = a.col_tiles - 1 - (rank * share + x % share);
+    return ctile >= 0;
+  }
+  const int item = x * a.per_xcd + rank;
   if (item >= a.kv_heads * a.col_tiles) return false;
   kvh = item / a.col_tiles;
   ctile = a.col_tiles - 1 - (item - kvh * a.col_tiles);
