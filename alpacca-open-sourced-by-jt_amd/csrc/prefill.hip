@@ -21,14 +21,16 @@
 // column tiles over many keys are cut along the keys as well
 // (prefill_split.hip, plan_split_prefill).
 //
-// Everything else (fp32, odd head dims, unaligned rows) runs the split-K
-// decode machinery in causal mode: query token t is a "sequence" whose
+// float32 chunks with the same head dims run prefill_f32 (prefill_f32.hip).
+// Everything else (odd head dims, unaligned rows, a few float32 tokens) runs
+// the split-K decode machinery in causal mode: query token t is a "sequence" whose
 // visible rows are those at absolute positions <= pos0 + t (inside the
 // window).
 #include <math.h>
 #include <string.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "alpx_common.h"
 #include "decode_internal.h"
@@ -168,6 +170,66 @@ SplitPlan plan_split_prefill(int q_tokens, int kv_tokens, int q_heads, int kv_he
   return p;
 }
 
+// float32 chunks: prefill_f32 over whole key ranges (splits 0), over pieces
+// of them, or (splits -1) the split-K decode machinery, one token per
+// "sequence", which is the faster one for a few tokens on a long prefix.
+// Estimated in us from measured times (32/8 heads, and 16/2 at head_dim
+// 256): two blocks on a CU walk a tile each in kTilePair, one block alone
+// in 0.6 of that; a split adds the combine (3 us, 6 at head_dim 256) and its
+// partials' bytes at 4 TB/s; the decode machinery takes kTokenRow per (token, kv head) and
+// cache row.  Measured, decode machinery / prefill_f32: head_dim 64, 1000
+// tokens on 0 rows 241 / 51, 100 on 4096 204 / 48 (8 pieces), 9 on 4096
+// 25 / 18 (32 pieces), 1 on 4096 12 / 12; head_dim 128, 1000 on 4096
+// 3325 / 599, 4 on 1024 22 / 16, 1 on 4096 16 / 25; head_dim 256, 700 on
+// 4096 1518 / 485 (4 pieces), 9 on 4096 33 / 42.
+SplitPlan plan_split_f32(int q_tokens, int kv_tokens, int kv_heads, int group, int head_dim,
+                         int rel0, int window) {
+  SplitPlan p = {0, 0, 0, 0};
+  const int rows = head_dim == 256 ? 16 : 32;
+  const double pair_us = head_dim == 64 ? 2.2 : (head_dim == 128 ? 4.1 : 4.4);
+  const double alone_us = 0.6 * pair_us;
+  const double token_row_us = head_dim == 64 ? 0.06e-3 : (head_dim == 128 ? 0.12e-3 : 0.3e-3);
+  const double combine_us = head_dim == 256 ? 6 : 3;
+  const int col_tiles = (int)(((int64_t)q_tokens * group + 63) / 64);
+  const int64_t items = (int64_t)col_tiles * kv_heads;
+  const int cus = 256;
+  const int first = host_tile_keys(q_tokens, kv_tokens, group, rel0, window, 64, rows, 0);
+  const int last =
+      host_tile_keys(q_tokens, kv_tokens, group, rel0, window, 64, rows, col_tiles - 1);
+  int most = std::max(1, std::max(first, last));
+  // a window's longest key range may be that of a tile in between
+  if (window > 0 && items < 2 * cus)
+    for (int ct = 1; ct < col_tiles - 1; ++ct)
+      most = std::max(most, host_tile_keys(q_tokens, kv_tokens, group, rel0, window, 64, rows, ct));
+  const double avg = std::max(1.0, 0.5 * (first + last));
+  const double decode_us =
+      3 + token_row_us * q_tokens * kv_heads * ((group + 15) / 16) * avg * rows;
+  auto walk_us = [&](double tiles, double blocks) {  // blocks of `tiles` key tiles each
+    const int per_cu = (int)std::ceil(blocks / cus);
+    return tiles * ((per_cu / 2) * pair_us + (per_cu % 2) * alone_us);
+  };
+  double best = std::max(most * alone_us, walk_us(avg, (double)items));
+  for (int pieces = 2; pieces <= 32 && items < 2 * cus; ++pieces) {
+    const int c = (most + pieces - 1) / pieces;
+    const int n = (most + c - 1) / c;
+    const double blocks = std::min<double>(items * (double)n, items * (avg / c + 0.5));
+    const double us = combine_us + blocks * 64 * head_dim * 8 / 4e6 + walk_us(c, blocks);
+    if (us < best) {
+      best = us;
+      p.splits = n;
+      p.split_tiles = c;
+    }
+  }
+  if (decode_us < 1.1 * best) {
+    p.splits = -1;
+  } else if (p.splits > 0) {
+    const size_t slots = (size_t)items * p.splits;
+    p.o_bytes = slots * 64 * head_dim * sizeof(float);
+    p.bytes = p.o_bytes + slots * 64 * sizeof(float2);
+  }
+  return p;
+}
+
 // Kernel choice for contiguous caches.  The paired kernel gains the tail a
 // heavy column tile runs alone and pays a second pipeline start (group 0)
 // and the final merge.  Same-box sweep (2048 query tokens, 32/8 or 16/2
@@ -227,16 +289,23 @@ PrefillKernelChoice choose_prefill(int q_tokens, int kv_tokens, int kv_heads, in
 // strides (`align` ORs their addresses and byte strides), and per-tile row
 // offsets that fit 32 bits.  Otherwise it takes the split-K path, which
 // needs a workspace of alpx_prefill_workspace_bytes.
-bool mfma_prefill_applies(int dtype, int key_dim, int value_dim, uintptr_t align,
-                          int64_t kv_tokens, int64_t k_pos_stride, int64_t v_pos_stride,
-                          int64_t rel0) {
+bool flash_operands(int dtype, int key_dim, int value_dim, uintptr_t align, int64_t kv_tokens,
+                    int64_t k_pos_stride, int64_t v_pos_stride, int64_t rel0) {
   const int64_t es = (int64_t)alpx::dtype_size(dtype);
-  return dtype != ALPX_F32 && key_dim == value_dim &&
+  return key_dim == value_dim &&
          (key_dim == 64 || key_dim == 128 || key_dim == 256) && (align & 15) == 0 &&
          alpx::override_value(ALPX_OVERRIDE_PREFILL_GENERIC) == 0 &&
          kv_tokens * k_pos_stride * es < ((int64_t)1 << 31) &&
          kv_tokens * v_pos_stride * es < ((int64_t)1 << 31) && rel0 < ((int64_t)1 << 30) &&
          rel0 > -((int64_t)1 << 30);
+}
+
+bool mfma_prefill_applies(int dtype, int key_dim, int value_dim, uintptr_t align,
+                          int64_t kv_tokens, int64_t k_pos_stride, int64_t v_pos_stride,
+                          int64_t rel0) {
+  return dtype != ALPX_F32 &&
+         flash_operands(dtype, key_dim, value_dim, align, kv_tokens, k_pos_stride, v_pos_stride,
+                        rel0);
 }
 
 // The query prologue a prefill forms itself (alpx_attention_layer_prefill
@@ -294,6 +363,39 @@ int prefill_impl(const void* q, const void* key, const void* value, const void* 
     return fail(ALPX_EUNSUPPORTED,
                 "alpx_prefill_causal_paged: needs fp16/bf16 pages, head_dim in {64, 128, 256}, "
                 "16-byte aligned rows and out_dtype == dtype");
+  PrefillArgs a = {};
+  a.kn = kn;
+  a.vn = vn;
+  a.new0 = (int)(q_pos0 - kv_start);
+  a.pages = pages;
+  a.page_shift = page_shift;
+  a.num_pages = num_pages;
+  a.ks_page = ((int64_t)1 << page_shift) * k_pos_stride;
+  a.vs_page = ((int64_t)1 << page_shift) * v_pos_stride;
+  a.q = q;
+  a.q_stride = q_stride;
+  if (qpro != nullptr) {
+    a.qw = qpro->qw;
+    a.q_rot = qpro->rot;
+    a.q_eps = qpro->eps;
+    a.q_R = qpro->R;
+  }
+  a.k = key;
+  a.v = value;
+  a.gate = gate;
+  a.gate_stride = gate_stride;
+  a.out = out;
+  a.ks_pos = k_pos_stride;
+  a.vs_pos = v_pos_stride;
+  a.pos0 = q_pos0;
+  a.kv_start = kv_start;
+  a.window = window;
+  a.q_tokens = q_tokens;
+  a.kv_tokens = kv_tokens;
+  a.q_heads = q_heads;
+  a.kv_heads = kv_heads;
+  a.group = group;
+  a.scale_log2 = scale * kLog2e;
   if (mfma) {
     const int cols_per_block = key_dim == 256 ? 64 : 128;
     const int tile_rows = key_dim == 256 ? 32 : 64;
@@ -313,6 +415,7 @@ int prefill_impl(const void* q, const void* key, const void* value, const void* 
       if (((uintptr_t)workspace & 15) != 0 || workspace_bytes < sp.bytes) sp.splits = 0;
     }
     const bool split = sp.splits > 0;
+    a.col_tiles = col_tiles;
     const void* kernel = nullptr;
     if (split)
       kernel = prefill_split_kernel(dtype, key_dim);
@@ -327,39 +430,6 @@ int prefill_impl(const void* q, const void* key, const void* value, const void* 
       kernel = pick_kernel_out<f16_t>(key_dim, out_dtype);
     else
       kernel = pick_kernel_out<bf16_t>(key_dim, out_dtype);
-    PrefillArgs a = {};
-    a.kn = kn;
-    a.vn = vn;
-    a.new0 = (int)(q_pos0 - kv_start);
-    a.pages = pages;
-    a.page_shift = page_shift;
-    a.num_pages = num_pages;
-    a.ks_page = ((int64_t)1 << page_shift) * k_pos_stride;
-    a.vs_page = ((int64_t)1 << page_shift) * v_pos_stride;
-    a.q = q;
-    a.q_stride = q_stride;
-    if (qpro != nullptr) {
-      a.qw = qpro->qw;
-      a.q_rot = qpro->rot;
-      a.q_eps = qpro->eps;
-      a.q_R = qpro->R;
-    }
-    a.k = key;
-    a.v = value;
-    a.gate = gate;
-    a.gate_stride = gate_stride;
-    a.out = out;
-    a.ks_pos = k_pos_stride;
-    a.vs_pos = v_pos_stride;
-    a.pos0 = q_pos0;
-    a.kv_start = kv_start;
-    a.window = window;
-    a.q_tokens = q_tokens;
-    a.kv_tokens = kv_tokens;
-    a.q_heads = q_heads;
-    a.kv_heads = kv_heads;
-    a.group = group;
-    a.col_tiles = col_tiles;
     const bool paired = pair || shared;  // a light and a heavy column tile per block
     const int64_t items =
         (int64_t)(paired ? (a.col_tiles + 1) / 2 : a.col_tiles) * kv_heads *
@@ -369,7 +439,6 @@ int prefill_impl(const void* q, const void* key, const void* value, const void* 
     a.part_o = (float*)workspace;
     a.part_st = (float2*)((char*)workspace + sp.o_bytes);
     a.per_xcd = (int)((items + kXcds - 1) / kXcds);
-    a.scale_log2 = scale * kLog2e;
     TimedRegion timed(ALPX_T_PREFILL, s);
     void* args[] = {(void*)&a};
     hipError_t err = hipLaunchKernel(kernel, dim3(a.per_xcd * kXcds), dim3(paired || split ? 512 : 256),
@@ -398,32 +467,61 @@ int prefill_impl(const void* q, const void* key, const void* value, const void* 
                                   q_pos0 - kv_start, nullptr, stream);
     if (rc != ALPX_OK) return rc;
   }
-  DecodeArgs a = {};
-  a.q = q;
-  a.k = key;
-  a.v = value;
-  a.seq_lens = nullptr;
-  a.gate = gate;  // the combine pass applies it ([token][head][d] = [b][h][d])
-  a.gate_stride = gate_stride;
-  a.out = out;
-  a.ks_pos = k_pos_stride;
-  a.ks_b = 0;
-  a.ks_h = key_dim;
-  a.vs_pos = v_pos_stride;
-  a.vs_b = 0;
-  a.vs_h = value_dim;
-  a.causal_pos0 = q_pos0;
-  a.kv_start = kv_start;
-  a.window = window;
-  a.length = kv_tokens;
-  a.batch = q_tokens;
-  a.q_heads = q_heads;
-  a.kv_heads = kv_heads;
-  a.group = group;
-  a.key_dim = key_dim;
-  a.value_dim = value_dim;
-  a.scale_log2 = scale * kLog2e;
-  return run_decode(a, dtype, out_dtype, workspace, workspace_bytes, s, ALPX_T_PREFILL,
+  if (dtype == ALPX_F32 && (int64_t)q_tokens * group < ((int64_t)1 << 30) &&
+      flash_operands(dtype, key_dim, value_dim, align, kv_tokens, k_pos_stride, v_pos_stride,
+                     q_pos0 - kv_start)) {
+    const SplitPlan sp = plan_split_f32(q_tokens, kv_tokens, kv_heads, group, key_dim,
+                                        (int)(q_pos0 - kv_start), window);
+    if (sp.splits >= 0 && ((uintptr_t)workspace & 15) == 0 && sp.bytes <= workspace_bytes) {
+      const bool split = sp.splits > 0;
+      a.col_tiles = (int)(((int64_t)q_tokens * group + 63) / 64);
+      a.splits = sp.splits;
+      a.split_tiles = sp.split_tiles;
+      a.part_o = (float*)workspace;
+      a.part_st = (float2*)((char*)workspace + sp.o_bytes);
+      const int64_t items = (int64_t)a.col_tiles * kv_heads * (split ? sp.splits : 1);
+      a.per_xcd = (int)((items + kXcds - 1) / kXcds);
+      void* args[] = {(void*)&a};
+      TimedRegion timed(ALPX_T_PREFILL, s);
+      hipError_t err = hipLaunchKernel(prefill_f32_kernel(key_dim, out_dtype, split),
+                                       dim3(a.per_xcd * kXcds), dim3(256), args, 0, s);
+      if (err != hipSuccess)
+        return fail(ALPX_EHIP, "prefill launch failed: %s", hipGetErrorString(err));
+      const int rc = check_launch("prefill_f32");
+      if (rc != ALPX_OK || !split) return rc;
+      err = hipLaunchKernel(prefill_combine_kernel(dtype, key_dim, out_dtype),
+                            dim3(a.col_tiles * kv_heads * 4), dim3(256), args, 0, s);
+      if (err != hipSuccess)
+        return fail(ALPX_EHIP, "prefill combine launch failed: %s", hipGetErrorString(err));
+      return check_launch("prefill_combine");
+    }
+  }
+  DecodeArgs d = {};
+  d.q = q;
+  d.k = key;
+  d.v = value;
+  d.seq_lens = nullptr;
+  d.gate = gate;  // the combine pass applies it ([token][head][d] = [b][h][d])
+  d.gate_stride = gate_stride;
+  d.out = out;
+  d.ks_pos = k_pos_stride;
+  d.ks_b = 0;
+  d.ks_h = key_dim;
+  d.vs_pos = v_pos_stride;
+  d.vs_b = 0;
+  d.vs_h = value_dim;
+  d.causal_pos0 = q_pos0;
+  d.kv_start = kv_start;
+  d.window = window;
+  d.length = kv_tokens;
+  d.batch = q_tokens;
+  d.q_heads = q_heads;
+  d.kv_heads = kv_heads;
+  d.group = group;
+  d.key_dim = key_dim;
+  d.value_dim = value_dim;
+  d.scale_log2 = scale * kLog2e;
+  return run_decode(d, dtype, out_dtype, workspace, workspace_bytes, s, ALPX_T_PREFILL,
                     ALPX_T_AUX);
 }
 

@@ -970,5 +970,6 @@ const void* prefill_pair_kernel(int dtype, int head_dim, int out_dtype);
 const void* prefill_shared_kernel(int dtype, int head_dim, int out_dtype);
 const void* prefill_split_kernel(int dtype, int head_dim);
 const void* prefill_combine_kernel(int dtype, int head_dim, int out_dtype);
+const void* prefill_f32_kernel(int head_dim, int out_dtype, bool split);
 
 }  // namespace alpx

@@ -68,6 +68,14 @@ prefill_split(PrefillArgs a) {
 // 16 columns), the O fragments of the 16 columns shared out over its four
 // waves.  Each piece weighs 2^(mc - M), M the largest offset among the
 // column's pieces that saw a key; the gate is applied before the rounding.
+template <typename T>
+__device__ __forceinline__ float gate_factor(T g) {
+  if constexpr (sizeof(T) == 4)
+    return stable_sigmoid(g);
+  else
+    return fast_sigmoid(to_f32(g));
+}
+
 template <typename T, typename TO, int D, int BK, int NQB>
 __global__ void __launch_bounds__(256)
 prefill_combine(PrefillArgs a) {
@@ -134,7 +142,7 @@ prefill_combine(PrefillArgs a) {
       const V4 g = *(const V4*)((const T*)a.gate + row * a.gate_stride + d0 + 16 * i);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        op[16 * i + e] = from_f32<TO>(o[i][e] * inv * fast_sigmoid(to_f32(g[e])));
+        op[16 * i + e] = from_f32<TO>(o[i][e] * inv * gate_factor<T>(g[e]));
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e) op[16 * i + e] = from_f32<TO>(o[i][e] * inv);
@@ -154,10 +162,11 @@ const void* pick_split(int D) {
 
 template <typename T, typename TO>
 const void* pick_combine(int D) {
+  constexpr bool f32 = sizeof(T) == 4;  // the tiles of prefill_f32
   switch (D) {
-    case 64: return (const void*)prefill_combine<T, TO, 64, 64, 2>;
-    case 128: return (const void*)prefill_combine<T, TO, 128, 64, 2>;
-    case 256: return (const void*)prefill_combine<T, TO, 256, 32, 1>;
+    case 64: return (const void*)prefill_combine<T, TO, 64, f32 ? 32 : 64, f32 ? 1 : 2>;
+    case 128: return (const void*)prefill_combine<T, TO, 128, f32 ? 32 : 64, f32 ? 1 : 2>;
+    case 256: return (const void*)prefill_combine<T, TO, 256, f32 ? 16 : 32, 1>;
   }
   return nullptr;
 }
@@ -178,6 +187,7 @@ const void* prefill_split_kernel(int dtype, int head_dim) {
 }
 
 const void* prefill_combine_kernel(int dtype, int head_dim, int out_dtype) {
+  if (dtype == ALPX_F32) return pick_combine_out<float>(head_dim, out_dtype);
   return dtype == ALPX_F16 ? pick_combine_out<f16_t>(head_dim, out_dtype)
                            : pick_combine_out<bf16_t>(head_dim, out_dtype);
 }

@@ -209,6 +209,48 @@ def test_prefill_split_matches_unsplit_and_oracle(gpu, ops, override, dtype, tq,
     assert np.abs(outs[0].cpu().numpy() - ref).max() <= TOL[dtype]
 
 
+@pytest.mark.parametrize("tq,prefix,hq,hkv,d,window,pos_off,gated,out", [
+    (70, 0, 8, 2, 64, 0, 0, False, "f32"), (130, 43, 6, 2, 128, 50, 0, True, "f32"),
+    (67, 0, 16, 2, 256, 0, 0, False, "f16"), (1100, 0, 3, 1, 64, 0, 0, False, "f32"),
+    (20, 1500, 8, 2, 64, 0, 0, False, "f32"), (33, 701, 12, 4, 128, 600, 0, True, "bf16"),
+    (50, 2001, 16, 2, 256, 0, 0, True, "f32"), (300, 0, 8, 8, 64, 0, -5, False, "f32"),
+    (363, 285, 2, 2, 256, 332, 0, False, "f32"), (500, 100, 4, 2, 64, 200, 0, False, "f32"),
+    (1, 4096, 4, 1, 128, 0, 0, False, "f32"), (9, 31, 40, 2, 128, 0, 0, False, "f32")])
+def test_prefill_f32_matches_oracle_and_decode_machinery(gpu, override, tq, prefix, hq, hkv, d,
+                                                         window, pos_off, gated, out):
+    """float32 chunks: whole key ranges, pieces of them merged by a second
+    launch, and the few tokens left to the decode machinery; key counts that
+    are no multiple of a tile, columns that do not fill a block, groups that
+    do not divide it, windows, rows that see no key, the gate, 16-bit
+    outputs.  Against the oracle, and against the decode machinery (the same
+    float32 products in another order: 2e-5, ten times what was seen)."""
+    import torch
+    P = _mod("_ops")
+    total = prefix + tq
+    rng = np.random.default_rng(tq + prefix + d)
+    r = lambda *s: rng.standard_normal(s).astype(np.float32)  # noqa: E731
+    q, K, V, gate = r(tq, hq, d), r(total, hkv, d), r(total, hkv, d), r(tq, hq, d)
+    pos0 = prefix if pos_off == 0 else 50 + pos_off
+    kv_start = 0 if pos_off == 0 else 50
+    outs = []
+    for generic in (0, 1):
+        override("prefill_generic", generic)
+        outs.append(P.prefill(_dev(torch, q, "f32", gpu), _dev(torch, K, "f32", gpu),
+                              _dev(torch, V, "f32", gpu), pos0=pos0, kv_start=kv_start,
+                              window=window, out_dtype=_tdtype(torch, out),
+                              gate=_dev(torch, gate, "f32", gpu) if gated else None).float())
+    ref = A.attention_batch(q, K, V, pos0 + np.arange(tq), hq // hkv, 1.0 / np.sqrt(d),
+                            window=window, kv_start=kv_start)
+    if gated:
+        ref = ref / (1.0 + np.exp(-gate))
+    got = outs[0].cpu().numpy()
+    assert np.abs(got - ref).max() <= TOL[out]
+    if out == "f32":
+        assert (outs[0] - outs[1]).abs().max().item() <= 2e-5
+    if pos_off < 0:
+        assert np.all(got[:-pos_off] == 0.0)
+
+
 def test_prefill_append_range_error_leaves_cache(gpu):
     import torch
     P = _mod("_ops")
