@@ -16,6 +16,7 @@ LIB_PATH = os.environ.get("ALPX_LIBRARY") or os.path.join(_HERE, "libalpx.so")
 ABI_VERSION = 1
 
 F32, F16, BF16 = 0, 1, 2
+F32_PLANES = 3  # float32 q / k as three bf16 planes per row (chunked GDN)
 OK, EINVAL, EUNSUPPORTED, EHIP, ERANGE = 0, -1, -2, -3, -4
 
 _c_int, _c_i64, _c_ptr, _c_size = ctypes.c_int, ctypes.c_int64, ctypes.c_void_p, ctypes.c_size_t

@@ -466,15 +466,17 @@ def prepare_gdn_step(state, q, k, v, beta, log_decay, out_dtype=None, out=None):
 
 def gdn_chunk(state, q, k, v, beta, log_decay, out_dtype=None):
     """GDN over ``T`` tokens in place on ``state``; q/k ``[B, T, Hk, Dk]``,
-    v ``[B, T, Hv, Dv]``, beta/log_decay ``[B, T, Hv]`` fp32.  Returns
-    ``[B, T, Hv, Dv]``."""
+    v ``[B, T, Hv, Dv]``, beta/log_decay ``[B, T, Hv]`` fp32; q/k may be
+    the plane fragments ``recurrent_prefill_prep(planes=True)`` returns, with
+    a batch axis (v fp32).  Returns ``[B, T, Hv, Dv]``."""
     torch = _torch()
     bsz, hv, dv, dk = (int(x) for x in state.shape)
-    tokens, hk = int(q.shape[1]), int(q.shape[2])
-    out = torch.empty((bsz, tokens, hv, dv), dtype=q.dtype if out_dtype is None else out_dtype,
+    planes = q.dim() == 7
+    tokens, hk = int(v.shape[1]), int(q.shape[1] if planes else q.shape[2])
+    out = torch.empty((bsz, tokens, hv, dv), dtype=v.dtype if out_dtype is None else out_dtype,
                       device=state.device)
     L = _lib.lib()
-    dtype = _lib.dtype_code(torch, q.dtype)
+    dtype = _lib.F32_PLANES if planes else _lib.dtype_code(torch, q.dtype)
     ws = None
     if L.alpx_gdn_chunk_uses_mfma(dtype, tokens, hk, hv, dk, dv):
         ws = _lib.workspace(torch, state.device,
@@ -809,7 +811,7 @@ def attention_layer_prefill(query_gate, key, value, q_norm, k_norm, key_cache, v
 
 def recurrent_prefill_prep(current, conv_weight, conv_history, beta_logits, alpha_logits,
                            dt_bias, ssm_a, *, key_heads, key_dim, value_heads, value_dim, eps,
-                           qkv_dtype, weight_layout="kc"):
+                           qkv_dtype, weight_layout="kc", planes=False):
     """Recurrent-layer inputs for ``T`` consecutive tokens of one sequence
     (all fp32 inputs): ``current [T, C]``, ``conv_history [K-1, C]`` (moved
     on in place).  Returns ``(q [T, Hk, Dk], k, v [T, Hv, Dv]`` in
@@ -823,7 +825,11 @@ def recurrent_prefill_prep(current, conv_weight, conv_history, beta_logits, alph
         kernel = int(conv_weight.shape[1])
         tap_stride, ch_stride = 1, kernel
     dev = current.device
-    q = torch.empty((tokens, int(key_heads), int(key_dim)), dtype=qkv_dtype, device=dev)
+    if planes:
+        q = torch.empty((int(key_heads), (tokens + 15) // 16, int(key_dim) // 32, 3, 64, 8),
+                        dtype=torch.bfloat16, device=dev)
+    else:
+        q = torch.empty((tokens, int(key_heads), int(key_dim)), dtype=qkv_dtype, device=dev)
     k = torch.empty_like(q)
     v = torch.empty((tokens, int(value_heads), int(value_dim)), dtype=qkv_dtype, device=dev)
     beta = torch.empty((tokens, int(value_heads)), dtype=torch.float32, device=dev)
@@ -834,7 +840,8 @@ def recurrent_prefill_prep(current, conv_weight, conv_history, beta_logits, alph
         beta_logits.data_ptr(), alpha_logits.data_ptr(), dt_bias.data_ptr(), ssm_a.data_ptr(),
         q.data_ptr(), k.data_ptr(), v.data_ptr(), beta.data_ptr(), g.data_ptr(), tokens,
         int(key_heads), int(value_heads), int(key_dim), int(value_dim), float(eps),
-        _lib.dtype_code(torch, qkv_dtype), _lib.stream_handle(torch, dev))
+        _lib.F32_PLANES if planes else _lib.dtype_code(torch, qkv_dtype),
+        _lib.stream_handle(torch, dev))
     _lib.check(rc)
     return q, k, v, beta, g
 

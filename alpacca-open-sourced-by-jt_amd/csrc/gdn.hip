@@ -187,13 +187,13 @@ gdn_step_kernel(GdnArgs a) {
 template <int N>
 __device__ __forceinline__ void split_planes8(const float* x, bf16x8 (&p)[N]) {
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    float r = x[j];
+  for (int j = 0; j < 8; j += 2) {
+    bf16x2 h[N];
+    split_planes2<N>(x[j], x[j + 1], h);
 #pragma unroll
     for (int n = 0; n < N; ++n) {
-      const bf16_t h = static_cast<bf16_t>(r);
-      p[n][j] = h;
-      if (n + 1 < N) r = r - static_cast<float>(h);
+      p[n][j] = h[n][0];
+      p[n][j + 1] = h[n][1];
     }
   }
 }
@@ -201,13 +201,13 @@ __device__ __forceinline__ void split_planes8(const float* x, bf16x8 (&p)[N]) {
 template <int N>
 __device__ __forceinline__ void split_planes4(f32x4 x, bf16x4 (&p)[N]) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    float r = x[j];
+  for (int j = 0; j < 4; j += 2) {
+    bf16x2 h[N];
+    split_planes2<N>(x[j], x[j + 1], h);
 #pragma unroll
     for (int n = 0; n < N; ++n) {
-      const bf16_t h = static_cast<bf16_t>(r);
-      p[n][j] = h;
-      if (n + 1 < N) r = r - static_cast<float>(h);
+      p[n][j] = h[n][0];
+      p[n][j + 1] = h[n][1];
     }
   }
 }
@@ -240,6 +240,17 @@ template <>
 struct Planes<float> {
   static constexpr int in = 3, der = 3;
 };
+// fp32 inputs whose q and k arrive already split (ALPX_F32_PLANES); v stays
+// fp32.
+template <>
+struct Planes<planes_t> {
+  static constexpr int in = 3, der = 3;
+};
+// Element types of v and of q / k.
+template <typename TI>
+using ValueT = typename std::conditional<std::is_same<TI, bf16_t>::value, bf16_t, float>::type;
+template <typename TI>
+using RowT = typename std::conditional<std::is_same<TI, float>::value, float, bf16_t>::type;
 
 // Rows in the order the transposing LDS read delivers them: k-slot j of
 // lane group `quad` is row 16 (j / 4) + 4 quad + j % 4.
@@ -294,6 +305,23 @@ __device__ __forceinline__ int tile_off(int mt, int ks, int lane) {
   return (tile_slot(mt, ks) * 64 + lane) * 8;
 }
 
+// Rows of 16-token tile `tile` (clamped to the last one) of key head kh in
+// the planes layout (ALPX_F32_PLANES): KS x 3 fragments of 64 lanes x 8.
+template <int DK>
+__device__ __forceinline__ const bf16_t* plane_rows(const GdnArgs& a, const void* x, int b, int kh,
+                                                    int tile) {
+  const int tiles = (a.T + 15) / 16;
+  return (const bf16_t*)x +
+         (((int64_t)b * a.Hk + kh) * tiles + min(tile, tiles - 1)) * (DK / 32 * 3 * 512);
+}
+// Row r and 16-byte unit cc of a chunk's unit idx, units in the layout's
+// order (tile, k step, lane).
+template <int KS>
+__device__ __forceinline__ void plane_unit(int idx, int& r, int& cc) {
+  r = 16 * (idx / (64 * KS)) + idx % 16;
+  cc = 4 * (idx % (64 * KS) / 64) + idx % 64 / 16;
+}
+
 // ------------------------------------------------------------ phase A
 
 // NG value heads of one key head per block (the value heads h with
@@ -306,6 +334,7 @@ template <typename TI, int DK, int NG>
 __global__ void __launch_bounds__(256 * NG)
 gdn_prep(GdnArgs a) {
   constexpr bool F32IN = std::is_same<TI, float>::value;
+  constexpr bool PL = std::is_same<TI, planes_t>::value;
   constexpr int NI = Planes<TI>::in, NS = Planes<TI>::der, ORD = NS - 1;
   constexpr int kS = DK + 8;   // bf16 LDS row stride
   constexpr int kF = kC + 4;   // fp32 LDS row stride
@@ -314,7 +343,7 @@ gdn_prep(GdnArgs a) {
   constexpr int kUPT = kC * kUnits / (256 * NG);
   static_assert(kUPT * 256 * NG == kC * kUnits, "K / Q rows must split evenly over the block");
   __shared__ __attribute__((aligned(16))) bf16_t Ks[NI][kC * kS];             // K rows
-  __shared__ __attribute__((aligned(16))) bf16_t Qs[F32IN ? 8 : kC * kS];     // Q rows
+  __shared__ __attribute__((aligned(16))) bf16_t Qs[NI > 1 ? 8 : kC * kS];    // Q rows
   // Per value head: diag(beta) A, then (per wave, its own 16 rows) M, P and
   // a staging tile; T; the block-recursion exchange; Gc; beta.
   __shared__ __attribute__((aligned(16))) float Bm_[NG][kC * kF];
@@ -340,7 +369,7 @@ gdn_prep(GdnArgs a) {
   // K, Q rows of the chunk, g and beta: every load reads a clamped row and
   // is issued before any is used, so they are all in flight together; rows
   // past the end are zeroed when stored.
-  bf16x8 kv[F32IN ? 1 : kUPT], qv[F32IN ? 1 : kUPT];
+  bf16x8 kv[F32IN ? 1 : kUPT][NI], qv[NI > 1 ? 1 : kUPT], qp[PL ? KS : 1][NI];
   f32x4 kf[F32IN ? kUPT : 1][2], qf[F32IN ? KS : 1][2];
   if constexpr (F32IN) {
 #pragma unroll
@@ -367,9 +396,23 @@ gdn_prep(GdnArgs a) {
     for (int u = 0; u < kUPT; ++u) {
       const int idx = u * 256 * NG + gtid;
       const int r = idx / kUnits, cc = idx - (idx / kUnits) * kUnits;
-      const int64_t off = (((int64_t)b * a.T + min(t0 + r, a.T - 1)) * a.Hk + kh) * DK + 8 * cc;
-      kv[u] = *(const bf16x8*)((const bf16_t*)a.k + off);
-      qv[u] = *(const bf16x8*)((const bf16_t*)a.q + off);
+      if constexpr (PL) {  // whole fragments: see plane_unit for r and cc
+        const bf16_t* p = plane_rows<DK>(a, a.k, b, kh, 4 * c + idx / (64 * KS)) +
+                          (idx % (64 * KS) / 64 * 3 * 64 + idx % 64) * 8;
+#pragma unroll
+        for (int n = 0; n < NI; ++n) kv[u][n] = *(const bf16x8*)(p + n * 512);
+      } else {
+        const int64_t off = (((int64_t)b * a.T + min(t0 + r, a.T - 1)) * a.Hk + kh) * DK + 8 * cc;
+        kv[u][0] = *(const bf16x8*)((const bf16_t*)a.k + off);
+        qv[u] = *(const bf16x8*)((const bf16_t*)a.q + off);
+      }
+    }
+    if constexpr (PL) {  // this wave's Q rows, A operands as they stand
+      const bf16_t* p = plane_rows<DK>(a, a.q, b, kh, 4 * c + wave) + lane * 8;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int n = 0; n < NI; ++n) qp[ks][n] = *(const bf16x8*)(p + (ks * 3 + n) * 512);
     }
   }
   const bool tok_ok = t0 + lane < a.T;
@@ -387,7 +430,8 @@ gdn_prep(GdnArgs a) {
 #pragma unroll
   for (int u = 0; u < kUPT; ++u) {
     const int idx = u * 256 * NG + gtid;
-    const int r = idx / kUnits, cc = idx - (idx / kUnits) * kUnits;
+    int r = idx / kUnits, cc = idx - (idx / kUnits) * kUnits;
+    if constexpr (PL) plane_unit<KS>(idx, r, cc);
     const bool ok = t0 + r < a.T;
     if constexpr (F32IN) {
       const float x[8] = {kf[u][0][0], kf[u][0][1], kf[u][0][2], kf[u][0][3],
@@ -397,8 +441,9 @@ gdn_prep(GdnArgs a) {
 #pragma unroll
       for (int n = 0; n < NI; ++n) *(bf16x8*)(Ks[n] + r * kS + 8 * cc) = ok ? pl[n] : zero8;
     } else {
-      *(bf16x8*)(Ks[0] + r * kS + 8 * cc) = ok ? kv[u] : zero8;
-      *(bf16x8*)(Qs + r * kS + 8 * cc) = ok ? qv[u] : zero8;
+#pragma unroll
+      for (int n = 0; n < NI; ++n) *(bf16x8*)(Ks[n] + r * kS + 8 * cc) = ok ? kv[u][n] : zero8;
+      if constexpr (!PL) *(bf16x8*)(Qs + r * kS + 8 * cc) = ok ? qv[u] : zero8;
     }
   }
   if (wave == 0) {
@@ -440,6 +485,9 @@ gdn_prep(GdnArgs a) {
           x[4 + j] = qok ? qf[ks][1][j] : 0.f;
         }
         split_planes8<NI>(x, qa);
+      } else if constexpr (PL) {
+#pragma unroll
+        for (int n = 0; n < NI; ++n) qa[n] = qok ? qp[ks][n] : zero8;
       } else {
         qa[0] = *(const bf16x8*)(Qs + (16 * wave + hl) * kS + 32 * ks + 8 * quad);
       }
@@ -649,11 +697,16 @@ __device__ __forceinline__ void apply_block(const GdnArgs& a, int& slice, int& h
   b = rest / a.Hv;
 }
 
-// Global inputs of one chunk, in three groups: what the K S^T / Q S^T step
-// reads as A operands (K and Q rows of the lane's token), the P and W
-// fragments of the wave's token rows, and the V rows and decays that waves
+// Global inputs of one chunk, in three groups: what the K S^T / Q S^T
+// products read as A operands (K and Q rows of the lane's token), the P and
+// W fragments of the wave's token rows, and the V rows and decays that waves
 // 0..2 stage in LDS for everyone.  fp32 inputs keep the loaded fp32 values
-// until their use, where they are split into planes.
+// until their use, where they are split into planes; a fragment of the
+// planes layout is one contiguous KiB per load.  (Rows cost more than their
+// bytes: a load of 16 of them touches a line per lane, about 32 cycles of
+// the CU's one load path against 16, and the fp32 kernel issues 39 KiB of
+// loads per wave and chunk.  C5 geometry, 1024 tokens, fp32: gdn_apply 75 us
+// from rows, 52 from fragments, same results.)
 template <typename TI, int DK>
 struct KqIn {
   bf16x8 k[DK / 32], q[DK / 32];
@@ -662,27 +715,21 @@ template <int DK>
 struct KqIn<float, DK> {
   f32x4 k[DK / 16], q[DK / 16];  // 32 ks + 8 quad + 0..3 in [2 ks], + 4..7 in [2 ks + 1]
 };
+template <int DK>
+struct KqIn<planes_t, DK> {
+  bf16x8 k[DK / 32][3], q[DK / 32][3];
+};
 template <int NS>
 struct PwIn {
   bf16x8 p[2][NS], w[2][NS];  // [k step][plane]
 };
-template <typename TI>
+// V rows and decays of one chunk, 16 or 32 bytes per lane: waves 0 and 1
+// hold V[token tid / 2][16-column slice half tid % 2], wave 2 (lanes 0..15)
+// Gc * log2(e) of tokens 4 lane .. 4 lane + 3, in x[0].
+template <typename TV>
 struct VgIn {
-  bf16x8 v;  // waves 0, 1: V[token tid / 2][16-column slice half tid % 2]
-  f32x4 g;   // wave 2, lanes 0..15: Gc * log2(e) of tokens 4 lane .. 4 lane + 3
+  u32x4 x[sizeof(TV) / 2];
 };
-// fp32 V: one pair of registers holds either a wave's V halves (waves 0,
-// 1) or the decays (wave 2, in v[0]), so no field is chosen by a branch
-// (a branch-selected field is stored through a selected pointer, in
-// scratch memory).
-template <>
-struct VgIn<float> {
-  f32x4 v[2];
-};
-__device__ __forceinline__ f32x4& vg_decay(VgIn<bf16_t>& in) { return in.g; }
-__device__ __forceinline__ f32x4& vg_decay(VgIn<float>& in) { return in.v[0]; }
-__device__ __forceinline__ const f32x4& vg_decay(const VgIn<bf16_t>& in) { return in.g; }
-__device__ __forceinline__ const f32x4& vg_decay(const VgIn<float>& in) { return in.v[0]; }
 
 // The planes of fp32 operand elements 8 j .. 8 j + 7 held as two f32x4.
 template <int N>
@@ -694,12 +741,15 @@ __device__ __forceinline__ void split_pair(const f32x4& x0, const f32x4& x1, bf1
 template <typename TI, typename TO, int DK>
 __global__ void __launch_bounds__(256)
 gdn_apply(GdnArgs a) {
-  constexpr bool F32IN = std::is_same<TI, float>::value;
+  typedef ValueT<TI> TV;
+  constexpr bool F32IN = std::is_same<TI, float>::value;  // q, k split here
+  constexpr bool PL = std::is_same<TI, planes_t>::value;  // q, k split by their producer
+  constexpr bool F32V = std::is_same<TV, float>::value;
   constexpr int NI = Planes<TI>::in, NS = Planes<TI>::der, ORD = NS - 1;
   constexpr int KS = DK / 32;
   constexpr int MT = DK / 64;     // state d tiles per wave
   // chunks of operands in flight (fp32 operands take twice the registers)
-  constexpr int PF = !F32IN && DK <= 128 ? 2 : 1;
+  constexpr int PF = !F32V && DK <= 128 ? 2 : 1;
   constexpr int kSB = DK + 8;     // bf16 row stride of the state planes
   // bf16 row stride of the K tile: 8 dwords past a multiple of 64 banks, so
   // the transposing reads of step (3) (four rows x four column groups per
@@ -713,12 +763,13 @@ gdn_apply(GdnArgs a) {
   __shared__ __attribute__((aligned(16))) bf16_t Kt[NI][kC * kSK];  // K [t][d]
   __shared__ __attribute__((aligned(16))) bf16_t Xp[NS][16 * kXB];  // X^T [r][t]
   __shared__ __attribute__((aligned(16))) bf16_t Yp[NS][16 * kXB];  // Y^T [r][t]
-  __shared__ __attribute__((aligned(16))) bf16_t Vs[F32IN ? 8 : kC * kVB];  // V [t][r]
-  __shared__ __attribute__((aligned(16))) float Vf[F32IN ? kC * kVF : 4];   // V [t][r], fp32
+  __shared__ __attribute__((aligned(16))) bf16_t Vs[F32V ? 8 : kC * kVB];   // V [t][r]
+  __shared__ __attribute__((aligned(16))) float Vf[F32V ? kC * kVF : 4];    // V [t][r], fp32
   __shared__ __attribute__((aligned(16))) TO Os[kC * kOB];      // O [t][r]
   __shared__ __attribute__((aligned(16))) float Gs[kC];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hl = lane & 15, quad = lane >> 4;
   int slice, h, b;
   apply_block(a, slice, h, b);
@@ -755,23 +806,32 @@ gdn_apply(GdnArgs a) {
   // the host also keeps below 2^32), so address arithmetic stays off the
   // quarter-rate 32 / 64-bit multiplies.
   const int krow = a.Hk * DK, vrow = a.Hv * a.Dv;
-  const TI* const kbase = (const TI*)a.k + (int64_t)b * a.T * krow + kh * DK + 8 * quad;
-  const TI* const qbase = (const TI*)a.q + (int64_t)b * a.T * krow + kh * DK + 8 * quad;
-  const TI* const vbase = (const TI*)a.v + (int64_t)b * a.T * vrow + h * a.Dv + r0;
+  const RowT<TI>* kbase = (const RowT<TI>*)a.k;
+  const RowT<TI>* qbase = (const RowT<TI>*)a.q;
+  if constexpr (!PL) {
+    kbase += (int64_t)b * a.T * krow + kh * DK + 8 * quad;
+    qbase += (int64_t)b * a.T * krow + kh * DK + 8 * quad;
+  }
+  const TV* const vbase = (const TV*)a.v + (int64_t)b * a.T * vrow + h * a.Dv + r0;
   TO* const obase = (TO*)a.out + (int64_t)b * a.T * vrow + h * a.Dv + r0;
   float* const wsbase = a.ws + bh * a.nchunks * ws_per_chunk<NS>();
-  auto fetch_kq = [&](KqIn<TI, DK>& in, int c) __attribute__((always_inline)) {
-    const unsigned off = __umul24((unsigned)min(c * kC + tw + hl, a.T - 1), (unsigned)krow);
+  auto fetch_rows = [&](auto& in, const RowT<TI>* base, int c) __attribute__((always_inline)) {
+    if constexpr (PL) {
+      const bf16_t* const p = plane_rows<DK>(a, base, b, kh, 4 * c + wave) + lane * 8;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      if constexpr (F32IN) {
-        in.k[2 * ks] = *(const f32x4*)(kbase + off + 32 * ks);
-        in.k[2 * ks + 1] = *(const f32x4*)(kbase + off + 32 * ks + 4);
-        in.q[2 * ks] = *(const f32x4*)(qbase + off + 32 * ks);
-        in.q[2 * ks + 1] = *(const f32x4*)(qbase + off + 32 * ks + 4);
-      } else {
-        in.k[ks] = *(const bf16x8*)(kbase + off + 32 * ks);
-        in.q[ks] = *(const bf16x8*)(qbase + off + 32 * ks);
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int n = 0; n < 3; ++n) in[ks][n] = *(const bf16x8*)(p + (ks * 3 + n) * 512);
+    } else {
+      const unsigned off = __umul24((unsigned)min(c * kC + tw + hl, a.T - 1), (unsigned)krow);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        if constexpr (F32IN) {
+          in[2 * ks] = *(const f32x4*)(base + off + 32 * ks);
+          in[2 * ks + 1] = *(const f32x4*)(base + off + 32 * ks + 4);
+        } else {
+          in[ks] = *(const bf16x8*)(base + off + 32 * ks);
+        }
       }
     }
   };
@@ -788,34 +848,30 @@ gdn_apply(GdnArgs a) {
       }
     }
   };
-  auto fetch_vg = [&](VgIn<TI>& in, int c) __attribute__((always_inline)) {
-    if (wave < 2) {
-      const unsigned t = (unsigned)min(c * kC + (tid >> 1), a.T - 1);
-      const TI* p = vbase + __umul24(t, (unsigned)vrow) + 8 * (tid & 1);
-      if constexpr (F32IN) {
-        in.v[0] = *(const f32x4*)p;
-        in.v[1] = *(const f32x4*)(p + 4);
-      } else {
-        in.v = *(const bf16x8*)p;
-      }
-    } else if (wave == 2 && lane < 16) {
-      vg_decay(in) = *(const f32x4*)(wsbase + c * (int)ws_per_chunk<NS>() + 4 * lane);
-    }
+  // One set of loads for every wave, from an address chosen per wave: with
+  // the loads on two sides of a branch, the address of one side shared a
+  // register with the other side's pending load and the wave waited there
+  // for every load in flight, this chunk's K rows among them (about 2 us per
+  // chunk with fp32 inputs).
+  auto fetch_vg = [&](VgIn<TV>& in, int c) __attribute__((always_inline)) {
+    const unsigned t = (unsigned)min(c * kC + (tid >> 1), a.T - 1);  // tid >= 128: unused
+    const char* const pv = (const char*)(vbase + __umul24(t, (unsigned)vrow) + 8 * (tid & 1));
+    const char* const pg =
+        (const char*)(wsbase + c * (int)ws_per_chunk<NS>() + 4 * (lane & 15));
+    const char* const p = wave < 2 ? pv : pg;
+#pragma unroll
+    for (int i = 0; i < (int)sizeof(TV) / 2; ++i) in.x[i] = *(const u32x4*)(p + 16 * i);
   };
-  auto stage_vg = [&](const VgIn<TI>& in, int c) __attribute__((always_inline)) {
+  auto stage_vg = [&](const VgIn<TV>& in, int c) __attribute__((always_inline)) {
     if (wave < 2) {
       const bool ok = c * kC + (tid >> 1) < a.T;
-      if constexpr (F32IN) {
-        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-        float* p = Vf + (tid >> 1) * kVF + 8 * (tid & 1);
-        *(f32x4*)p = ok ? in.v[0] : zero;
-        *(f32x4*)(p + 4) = ok ? in.v[1] : zero;
-      } else {
-        const bf16x8 zero = {};
-        *(bf16x8*)(Vs + (tid >> 1) * kVB + 8 * (tid & 1)) = ok ? in.v : zero;
-      }
+      TV* const p = F32V ? (TV*)Vf + (tid >> 1) * kVF + 8 * (tid & 1)
+                         : (TV*)Vs + (tid >> 1) * kVB + 8 * (tid & 1);
+#pragma unroll
+      for (int i = 0; i < (int)sizeof(TV) / 2; ++i)
+        *(u32x4*)((char*)p + 16 * i) = ok ? in.x[i] : (u32x4){0u, 0u, 0u, 0u};
     } else if (wave == 2 && lane < 16) {
-      *(f32x4*)(Gs + 4 * lane) = vg_decay(in);
+      *(u32x4*)(Gs + 4 * lane) = in.x[0];
     }
   };
   // Output tile of chunk c (staged in LDS) -> global, 16 bytes per lane.
@@ -838,12 +894,13 @@ gdn_apply(GdnArgs a) {
   // than branching.
   KqIn<TI, DK> kq[PF];
   PwIn<NS> pw[PF];
-  VgIn<TI> vg[PF];
+  VgIn<TV> vg[PF];
 #pragma unroll
   for (int p = 0; p < PF; ++p) {
     const int c = min(p, a.nchunks - 1);
     fetch_vg(vg[p], c);
-    fetch_kq(kq[p], c);
+    fetch_rows(kq[p].k, kbase, c);
+    fetch_rows(kq[p].q, qbase, c);
     fetch_pw(pw[p], c);
   }
   put_state();
@@ -851,12 +908,19 @@ gdn_apply(GdnArgs a) {
   fetch_vg(vg[0], min(PF, a.nchunks - 1));
   __syncthreads();
 
-  auto chunk = [&](int c, KqIn<TI, DK>& kqc, PwIn<NS>& pwc, VgIn<TI>& vgn)
+  auto chunk = [&](int c, KqIn<TI, DK>& kqc, PwIn<NS>& pwc, VgIn<TV>& vgn)
                    __attribute__((always_inline)) {
     const int t0 = c * kC;
     const int cf = min(c + PF, a.nchunks - 1);
 
-    // (1) K S^T and Q S^T for this wave's tokens (B = S^T: lane holds
+    // One wave per SIMD: what a step waits for (its LDS reads, the other
+    // waves at the barrier) is time lost unless other work of the wave
+    // stands there.  So the output's products, which nothing waits for, run
+    // behind a step's first LDS reads (Q S^T in step (2), P X^T in step
+    // (3)), and a chunk's global loads are issued a third per step, each
+    // behind the products that free their registers.
+    //
+    // (1) K S^T for this wave's tokens (B = S^T: lane holds
     // S[r0 + hl][32 ks + 8 quad + 0..7]); X^T = V - diag(exp Gc) K S^T.  The
     // wave's K rows also go to the K tile for step (3).
     bf16x8 sp[KS][NS];
@@ -864,38 +928,26 @@ gdn_apply(GdnArgs a) {
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
       for (int n = 0; n < NS; ++n) sp[ks][n] = *(const bf16x8*)(Sp[n] + hl * kSB + 32 * ks + 8 * quad);
+    // The previous chunk's output tile goes out while the reads run.
+    if (c > 0) flush_out(c - 1);
     f32x4 kst = {0.f, 0.f, 0.f, 0.f}, qst = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       bf16x8 kp[NI];
       if constexpr (F32IN) {
         split_pair<NI>(kqc.k[2 * ks], kqc.k[2 * ks + 1], kp);
+      } else if constexpr (PL) {
 #pragma unroll
-        for (int n = 0; n < NI; ++n) *(bf16x8*)(Kt[n] + (tw + hl) * kSK + 32 * ks + 8 * quad) = kp[n];
+        for (int n = 0; n < NI; ++n) kp[n] = kqc.k[ks][n];
       } else {
         kp[0] = kqc.k[ks];
       }
+#pragma unroll
+      for (int n = 0; n < NI; ++n) *(bf16x8*)(Kt[n] + (tw + hl) * kSK + 32 * ks + 8 * quad) = kp[n];
       kst = mfma_planes<NI, NS, ORD>(kp, sp[ks], kst);
     }
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      bf16x8 qp[NI];
-      if constexpr (F32IN)
-        split_pair<NI>(kqc.q[2 * ks], kqc.q[2 * ks + 1], qp);
-      else
-        qp[0] = kqc.q[ks];
-      qst = mfma_planes<NI, NS, ORD>(qp, sp[ks], qst);
-    }
-    // The previous chunk's output tile goes out while the products run.
-    if (c > 0) flush_out(c - 1);
-    if constexpr (!F32IN) {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        *(bf16x8*)(Kt[0] + (tw + hl) * kSK + 32 * ks + 8 * quad) = kqc.k[ks];
-    }
-    fetch_kq(kqc, cf);
     f32x4 v4;
-    if constexpr (F32IN) {
+    if constexpr (F32V) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) v4[e] = Vf[(tw + 4 * quad + e) * kVF + hl];
     } else {
@@ -919,22 +971,35 @@ gdn_apply(GdnArgs a) {
       for (int n = 0; n < NS; ++n) *(bf16x4*)(Xp[n] + hl * kXB + tw + 4 * quad) = pl[n];
     }
     __syncthreads();  // X^T and the K tile complete; every wave has read S, V and Gc
+    __builtin_amdgcn_sched_barrier(0);
 
-    // (2) Y^T = W X^T and O = scale exp(Gc) Q S^T + P X^T for this wave's
-    // tokens (W and P are causal: waves 0 and 1, tokens < 32, skip tokens
-    // 32..63).
+    // (2) Y^T = W X^T for this wave's tokens (W and P are causal: waves 0
+    // and 1, tokens < 32, skip tokens 32..63), Q S^T behind X's reads.
     bf16x8 xp[2][NS];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
       for (int n = 0; n < NS; ++n) xp[ks][n] = *(const bf16x8*)(Xp[n] + hl * kXB + 32 * ks + 8 * quad);
-    f32x4 yt = {0.f, 0.f, 0.f, 0.f}, po = {0.f, 0.f, 0.f, 0.f};
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      bf16x8 qp[NI];
+      if constexpr (F32IN) {
+        split_pair<NI>(kqc.q[2 * ks], kqc.q[2 * ks + 1], qp);
+      } else if constexpr (PL) {
+#pragma unroll
+        for (int n = 0; n < NI; ++n) qp[n] = kqc.q[ks][n];
+      } else {
+        qp[0] = kqc.q[ks];
+      }
+      qst = mfma_planes<NI, NS, ORD>(qp, sp[ks], qst);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_rows(kqc.k, kbase, cf);
+    f32x4 yt = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
       if (tile_live(wave, ks)) yt = mfma_planes<NS, NS, ORD>(pwc.w[ks], xp[ks], yt);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-      if (tile_live(wave, ks)) po = mfma_planes<NS, NS, ORD>(pwc.p[ks], xp[ks], po);
     {
       bf16x4 pl[NS];
       split_planes4<NS>(yt, pl);
@@ -943,14 +1008,13 @@ gdn_apply(GdnArgs a) {
     }
     stage_vg(vgn, c + 1);
     fetch_vg(vgn, min(c + 1 + PF, a.nchunks - 1));
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      Os[(tw + 4 * quad + e) * kOB + hl] = from_f32<TO>(a.scale * gam[e] * qst[e] + po[e]);
-    __syncthreads();  // Y^T, the output tile, V and Gc of the next chunk complete
+    __syncthreads();  // Y^T, V and Gc of the next chunk complete
+    __builtin_amdgcn_sched_barrier(0);
 
     // (3) S^T <- exp(Gc_last) S^T + K^T Y^T: A = K^T through the transposing
     // read (k-slot j of lane group quad is token 32 ks + tr_slot(quad, j)),
-    // B = Y^T in the same token order; then publish the new state.
+    // B = Y^T in the same token order; then publish the new state.  Behind
+    // the reads, O = scale exp(Gc) Q S^T + P X^T.
     bf16x8 yp[2][NS];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -961,6 +1025,12 @@ gdn_apply(GdnArgs a) {
         yp[ks][n] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 po = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      if (tile_live(wave, ks)) po = mfma_planes<NS, NS, ORD>(pwc.p[ks], xp[ks], po);
+    fetch_rows(kqc.q, qbase, cf);
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
       const int mt = wave + 4 * i;
@@ -978,11 +1048,13 @@ gdn_apply(GdnArgs a) {
       }
       sown[i] = acc;
     }
-    // P and W of chunk c + PF: issued here rather than with step (2)'s
-    // other loads, so each step issues about a third of the chunk's loads.
-    fetch_pw(pwc, cf);
     put_state();
-    __syncthreads();  // new state published; every wave has read Y^T and the K tile
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      Os[(tw + 4 * quad + e) * kOB + hl] = from_f32<TO>(a.scale * gam[e] * qst[e] + po[e]);
+    fetch_pw(pwc, cf);
+    __syncthreads();  // new state and the output tile complete; Y^T and the K tile are read
+    __builtin_amdgcn_sched_barrier(0);
   };
 
   for (int c0 = 0; c0 < a.nchunks; c0 += PF) {
@@ -1000,7 +1072,7 @@ int launch_chunk(const GdnArgs& a, hipStream_t s) {
   // two value heads per phase-A block where the key head has an even
   // number of them; fp32 inputs at head_dim 256 stage three K planes, which
   // leave LDS for one head's matrices only
-  constexpr bool kPairs = !(std::is_same<TI, float>::value && DK == 256);
+  constexpr bool kPairs = !(Planes<TI>::in > 1 && DK == 256);
   if constexpr (kPairs) {
     if ((a.Hv / a.Hk) % 2 == 0) {
       hipLaunchKernelGGL((gdn_prep<TI, DK, 2>), dim3(a.nchunks, a.Hv / 2, a.B), dim3(512), 0, s,
@@ -1139,7 +1211,7 @@ extern "C" int alpx_gdn_chunk_uses_mfma(int dtype, int tokens, int key_heads, in
   // products: token < 2^24, row < 2^24 and token x row < 2^32
   const bool offsets_fit = tokens < (1 << 24) && krow < (1 << 24) && vrow < (1 << 24) &&
                            (int64_t)tokens * (krow > vrow ? krow : vrow) <= (int64_t)UINT32_MAX;
-  return (dtype == ALPX_BF16 || dtype == ALPX_F32) &&
+  return (dtype == ALPX_BF16 || dtype == ALPX_F32 || dtype == ALPX_F32_PLANES) &&
                  (key_dim == 64 || key_dim == 128 || key_dim == 256) && value_dim % 16 == 0 &&
                  offsets_fit && override_value(ALPX_OVERRIDE_GDN_SEQUENTIAL) == 0
              ? 1
@@ -1162,7 +1234,8 @@ extern "C" int alpx_gdn_chunk_prefill(float* state, const void* q, const void* k
                                       int value_dim, int dtype, int out_dtype, void* stream) {
   using namespace alpx;
   int rc = validate(state, q, k, v, beta, log_decay, out, batch, key_heads, value_heads, key_dim,
-                    value_dim, dtype, out_dtype, "alpx_gdn_chunk_prefill");
+                    value_dim, dtype == ALPX_F32_PLANES ? ALPX_F32 : dtype, out_dtype,
+                    "alpx_gdn_chunk_prefill");
   if (rc != ALPX_OK) return rc;
   if (tokens <= 0) return fail(ALPX_EINVAL, "alpx_gdn_chunk_prefill: tokens must be positive");
   hipStream_t s = (hipStream_t)stream;
@@ -1194,9 +1267,14 @@ extern "C" int alpx_gdn_chunk_prefill(float* state, const void* q, const void* k
       return fail(ALPX_EINVAL, "alpx_gdn_chunk_prefill: workspace holds %zu bytes, needs %zu",
                   workspace_bytes, need);
     a.ws = (float*)workspace;
+    if (dtype == ALPX_F32_PLANES) return launch_chunk_ti<planes_t>(a, out_dtype, s);
     return dtype == ALPX_F32 ? launch_chunk_ti<float>(a, out_dtype, s)
                              : launch_chunk_ti<bf16_t>(a, out_dtype, s);
   }
+  if (dtype == ALPX_F32_PLANES)
+    return fail(ALPX_EUNSUPPORTED,
+                "alpx_gdn_chunk_prefill: split q and k need the chunked kernels' sizes and 16-byte "
+                "aligned buffers");
   // Token-sequential form (fp16 inputs, other shapes): the decode step per
   // token, exactly the reference's recurrence order.
   const size_t es = dtype_size(dtype);

@@ -757,7 +757,7 @@ __global__ void __launch_bounds__(256) recurrent_finish_kernel(FinishArgs f) {
 struct ChunkPrepArgs {
   const float* x;     // [T, C] convolution inputs of T consecutive tokens
   const float* w;     // conv weights, tap i / channel c at i * w_tap + c * w_ch
-  const float* hist;  // [K - 1, C] history before token 0 (row 0 oldest)
+  float* hist;        // [K - 1, C] history before token 0 (row 0 oldest); the tiled form moves it on
   const float* bl;    // [T, Hv]
   const float* al;    // [T, Hv]
   const float* dtb;   // [Hv]
@@ -772,9 +772,27 @@ struct ChunkPrepArgs {
   float eps;
 };
 
+// Outputs of a chunk prep to TO: q / k and v elements (planes_t: q / k as
+// the fragments of three bf16 planes, ALPX_F32_PLANES, v fp32).
+template <typename TO>
+constexpr bool kPlanes = std::is_same<TO, planes_t>::value;
+template <typename TO>
+using QkT = typename std::conditional<kPlanes<TO>, bf16_t, TO>::type;
+template <typename TO>
+using ValT = typename std::conditional<kPlanes<TO>, float, TO>::type;
+
+// Element offset of channel i of token t of key head j in the planes layout:
+// [head][16-token tile][k step of 32][plane][lane 16 quad + row][8], plane 0.
+// Its rows past the last token, up to the tile's end, are zeros.
+__device__ __forceinline__ int64_t plane_offset(int T, int Dk, int j, int t, int i) {
+  const int64_t tile = (int64_t)j * ((T + 15) / 16) + t / 16;
+  return ((tile * (Dk / 32) + i / 32) * 3 * 64 + (i % 32 / 8 * 16 + t % 16)) * 8 + i % 8;
+}
+__host__ __device__ __forceinline__ int padded_tokens(int T) { return (T + 15) / 16 * 16; }
+
 // One wave per (token, head slot), as recurrent_prep_kernel, with token t's
 // convolution window taken from the extended sequence E = [history; x]:
-// tap i reads E row t + i (tap K - 1 is x[t]).  The history is read only;
+// tap i reads E row t + i (tap K - 1 is x[t]).  The history is only read;
 // conv_history_advance moves it on afterwards.
 template <typename TO>
 __global__ void __launch_bounds__(256) recurrent_chunk_prep_kernel(ChunkPrepArgs a) {
@@ -782,22 +800,31 @@ __global__ void __launch_bounds__(256) recurrent_chunk_prep_kernel(ChunkPrepArgs
   const int lane = threadIdx.x & 63;
   const int slots = 2 * a.Hk + a.Hv;
   const int64_t id = (int64_t)blockIdx.x * 4 + wave;
-  if (id >= (int64_t)a.T * slots) return;
+  const int tokens = kPlanes<TO> ? padded_tokens(a.T) : a.T;
+  if (id >= (int64_t)tokens * slots) return;
   const int t = (int)(id / slots);
   const int j = (int)(id - (int64_t)t * slots);
+  if (kPlanes<TO> && t >= a.T) {  // a padding row of the planes layout
+    bf16_t* const p = (bf16_t*)(j < a.Hk ? a.q : a.k);
+    for (int i = lane; j < 2 * a.Hk && i < a.Dk; i += 64)
+      for (int m = 0; m < 3; ++m)
+        p[plane_offset(a.T, a.Dk, j % a.Hk, t, i) + m * 512] = from_f32<bf16_t>(0.f);
+    return;
+  }
   const int C = 2 * a.Hk * a.Dk + a.Hv * a.Dv;
   int c0, n;
-  TO* dst;
+  QkT<TO>* dst = nullptr;
+  ValT<TO>* vdst = nullptr;
   if (j < 2 * a.Hk) {
     c0 = j * a.Dk;
     n = a.Dk;
-    dst = j < a.Hk ? (TO*)a.q + ((int64_t)t * a.Hk + j) * a.Dk
-                   : (TO*)a.k + ((int64_t)t * a.Hk + (j - a.Hk)) * a.Dk;
+    dst = (QkT<TO>*)(j < a.Hk ? a.q : a.k);
+    if (!kPlanes<TO>) dst += ((int64_t)t * a.Hk + j % a.Hk) * a.Dk;
   } else {
     const int h = j - 2 * a.Hk;
     c0 = 2 * a.Hk * a.Dk + h * a.Dv;
     n = a.Dv;
-    dst = (TO*)a.v + ((int64_t)t * a.Hv + h) * a.Dv;
+    vdst = (ValT<TO>*)a.v + ((int64_t)t * a.Hv + h) * a.Dv;
     if (lane == 0) {
       const int64_t th = (int64_t)t * a.Hv + h;
       a.beta[th] = stable_sigmoid(a.bl[th]);
@@ -847,7 +874,23 @@ __global__ void __launch_bounds__(256) recurrent_chunk_prep_kernel(ChunkPrepArgs
 #pragma unroll
   for (int e = 0; e < kPer; ++e) {
     const int i = lane + 64 * e;
-    if (i < n) dst[i] = from_f32<TO>(j < 2 * a.Hk ? y[e] * inv : y[e]);
+    if (i >= n) continue;
+    if (j >= 2 * a.Hk) {
+      vdst[i] = from_f32<ValT<TO>>(y[e]);
+    } else if constexpr (kPlanes<TO>) {
+      // the product rounded first, as it is stored in the other forms
+      float x;
+      {
+#pragma clang fp contract(off)
+        x = y[e] * inv;
+      }
+      bf16x2 p[3];
+      split_planes2<3>(x, 0.f, p);
+#pragma unroll
+      for (int m = 0; m < 3; ++m) dst[plane_offset(a.T, n, j % a.Hk, t, i) + m * 512] = p[m][0];
+    } else {
+      dst[i] = from_f32<QkT<TO>>(y[e] * inv);
+    }
   }
 }
 
@@ -885,18 +928,20 @@ __global__ void __launch_bounds__(256) recurrent_chunk_prep_tile(ChunkPrepArgs a
   const int C = 2 * a.Hk * a.Dk + a.Hv * a.Dv;
   const bool is_qk = j < 2 * a.Hk;
   int c0, n;
-  TO* dst;
+  QkT<TO>* dst = nullptr;
+  ValT<TO>* vdst = nullptr;
   int64_t dstride;
   if (is_qk) {
     c0 = j * a.Dk;
     n = a.Dk;
-    dst = j < a.Hk ? (TO*)a.q + (int64_t)j * a.Dk : (TO*)a.k + (int64_t)(j - a.Hk) * a.Dk;
+    dst = (QkT<TO>*)(j < a.Hk ? a.q : a.k);
+    if (!kPlanes<TO>) dst += (int64_t)(j % a.Hk) * a.Dk;
     dstride = (int64_t)a.Hk * a.Dk;
   } else {
     const int h = j - 2 * a.Hk;
     c0 = 2 * a.Hk * a.Dk + h * a.Dv;
     n = a.Dv;
-    dst = (TO*)a.v + (int64_t)h * a.Dv;
+    vdst = (ValT<TO>*)a.v + (int64_t)h * a.Dv;
     dstride = (int64_t)a.Hv * a.Dv;
     if (tid < kTileTokens && t0 + tid < a.T) {
       const int64_t th = (int64_t)(t0 + tid) * a.Hv + h;
@@ -932,6 +977,29 @@ __global__ void __launch_bounds__(256) recurrent_chunk_prep_tile(ChunkPrepArgs a
       win[r] = *(const f32x4*)src;
     }
   }
+  // The history after the chunk, rows T .. T + K - 2 of E.  Only this
+  // thread reads these channels' history (P >= K - 1, so tokens tb >= P see
+  // none of it), and it has: no other launch has to move it on.
+  if (tb == 0 && act) {
+    f32x4 last[kTileTaps - 1];
+#pragma unroll
+    for (int r = 0; r < kTileTaps - 1; ++r) {
+      const int er = a.T + r;
+      if (r + 1 < K) {
+        if (er >= K - 1) {
+          last[r] = *(const f32x4*)(a.x + (int64_t)(er - (K - 1)) * C + c);
+        } else {  // er < K - 1 <= 3: still the old history
+          last[r] = win[0];
+#pragma unroll
+          for (int o = 1; o < kTileTaps - 1; ++o)
+            if (o == er) last[r] = win[o];
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < kTileTaps - 1; ++r)
+      if (r + 1 < K) *(f32x4*)(a.hist + (int64_t)r * C + c) = last[r];
+  }
 #pragma unroll
   for (int p = 0; p < kMaxP; ++p) {
     if (p < P) {
@@ -954,7 +1022,53 @@ __global__ void __launch_bounds__(256) recurrent_chunk_prep_tile(ChunkPrepArgs a
         for (int e = 0; e < 4; ++e) y[e] *= inv;
       }
       const int t = tb + p;
-      if (act && t < a.T) store4(dst + (int64_t)t * dstride + 4 * cg, y);
+      if constexpr (kPlanes<TO>) {
+        if (is_qk) {  // kept (in the window row no later token needs) for the fragments
+          const bool ok = t < a.T;
+          win[p] = (f32x4){ok ? y[0] : 0.f, ok ? y[1] : 0.f, ok ? y[2] : 0.f, ok ? y[3] : 0.f};
+          continue;
+        }
+      }
+      if (!act || t >= a.T) continue;
+      if (is_qk)
+        store4(dst + (int64_t)t * dstride + 4 * cg, y);
+      else
+        store4(vdst + (int64_t)t * dstride + 4 * cg, y);
+    }
+  }
+  if constexpr (kPlanes<TO>) {
+    if (!is_qk) return;
+    // One plane at a time through LDS rows (padded by 16 bytes, so neither
+    // the row writes nor the fragment reads share banks): the fragments go
+    // out as whole 1 KiB stores.  Stored straight from the channel groups,
+    // 8 bytes per lane and 256 apart, they took the kernel from 18 to 30 us
+    // (1024 tokens, 16 + 16 heads of 128, 32 value heads).
+    extern __shared__ __attribute__((aligned(16))) bf16_t rows[];
+    const int stride = n + 8, ksn = n / 32;
+    const int wave = tid >> 6, lane = tid & 63;
+    const int tiles = (a.T + 15) / 16;
+    for (int m = 0; m < 3; ++m) {
+#pragma unroll
+      for (int p = 0; p < kMaxP; ++p) {
+        if (p < P) {
+          bf16x2 h0[1], h1[1];
+          split_planes2<1>(win[p][0], win[p][1], h0);
+          split_planes2<1>(win[p][2], win[p][3], h1);
+          const bf16x4 h = __builtin_shufflevector(h0[0], h1[0], 0, 1, 2, 3);
+          win[p] = win[p] - __builtin_convertvector(h, f32x4);
+          if (act) *(bf16x4*)(rows + (tg * P + p) * stride + 4 * cg) = h;
+        }
+      }
+      __syncthreads();
+      for (int f = wave; f < 4 * ksn; f += 4) {
+        const int tile = f / ksn, ks = f - tile * ksn, gt = t0 / 16 + tile;
+        if (gt >= tiles) continue;
+        const u32x4 x = *(const u32x4*)(rows + (16 * tile + (lane & 15)) * stride + 32 * ks +
+                                        8 * (lane >> 4));
+        *(u32x4*)(dst + (((int64_t)(j % a.Hk) * tiles + gt) * ksn + ks) * 1536 + m * 512 +
+                  lane * 8) = x;
+      }
+      __syncthreads();
     }
   }
 }
@@ -1508,13 +1622,17 @@ extern "C" int alpx_recurrent_prefill_prep(const float* current, const float* co
       !alpha_logits || !dt_bias || !ssm_a || !q_out || !k_out || !v_out || !beta_out ||
       !log_decay_out)
     return fail(ALPX_EINVAL, "alpx_recurrent_prefill_prep: null buffer");
-  if (!dtype_ok(out_dtype)) return fail(ALPX_EINVAL, "alpx_recurrent_prefill_prep: unknown dtype");
+  if (!dtype_ok(out_dtype) && out_dtype != ALPX_F32_PLANES)
+    return fail(ALPX_EINVAL, "alpx_recurrent_prefill_prep: unknown dtype");
   if (tokens <= 0 || key_heads <= 0 || value_heads <= 0 || key_dim <= 0 || value_dim <= 0 ||
       conv_kernel <= 0)
     return fail(ALPX_EINVAL, "alpx_recurrent_prefill_prep: sizes must be positive");
   if (value_heads % key_heads != 0) return fail(ALPX_EINVAL, "GDN value heads must be a multiple of key heads");
   if (key_dim > kMaxDim || value_dim > kMaxDim)
     return fail(ALPX_EUNSUPPORTED, "alpx_recurrent_prefill_prep: head dims above %d", kMaxDim);
+  if (out_dtype == ALPX_F32_PLANES && key_dim % 32 != 0)
+    return fail(ALPX_EUNSUPPORTED,
+                "alpx_recurrent_prefill_prep: split q and k need a key_dim in multiples of 32");
   if (!(eps > 0.f) || !isfinite(eps)) return fail(ALPX_EINVAL, "epsilon must be positive and finite");
   ChunkPrepArgs a;
   a.x = current;
@@ -1541,7 +1659,7 @@ extern "C" int alpx_recurrent_prefill_prep(const float* current, const float* co
   hipStream_t s = (hipStream_t)stream;
   TimedRegion timed(ALPX_T_LAYER, s);
   const int slots = 2 * key_heads + value_heads;
-  const size_t osz = dtype_size(out_dtype);
+  const size_t osz = out_dtype == ALPX_F32_PLANES ? 4 : dtype_size(out_dtype);
   const bool tiled = conv_kernel <= kTileTaps && key_dim % 4 == 0 && value_dim % 4 == 0 &&
                      key_dim <= 256 && value_dim <= 256 && aligned(current, 16) &&
                      (conv_kernel == 1 || aligned(conv_history, 16)) &&
@@ -1551,19 +1669,27 @@ extern "C" int alpx_recurrent_prefill_prep(const float* current, const float* co
     switch (out_dtype) {
       case ALPX_F32: hipLaunchKernelGGL(recurrent_chunk_prep_tile<float>, grid, dim3(256), 0, s, a); break;
       case ALPX_F16: hipLaunchKernelGGL(recurrent_chunk_prep_tile<f16_t>, grid, dim3(256), 0, s, a); break;
+      case ALPX_F32_PLANES:
+        hipLaunchKernelGGL(recurrent_chunk_prep_tile<planes_t>, grid, dim3(256),
+                           kTileTokens * (key_dim + 8) * sizeof(bf16_t), s, a);
+        break;
       default: hipLaunchKernelGGL(recurrent_chunk_prep_tile<bf16_t>, grid, dim3(256), 0, s, a); break;
     }
   } else {
-    const int64_t waves = (int64_t)tokens * slots;
+    const int rows = out_dtype == ALPX_F32_PLANES ? padded_tokens(tokens) : tokens;
+    const int64_t waves = (int64_t)rows * slots;
     const dim3 grid((unsigned)((waves + 3) / 4));
     switch (out_dtype) {
       case ALPX_F32: hipLaunchKernelGGL(recurrent_chunk_prep_kernel<float>, grid, dim3(256), 0, s, a); break;
       case ALPX_F16: hipLaunchKernelGGL(recurrent_chunk_prep_kernel<f16_t>, grid, dim3(256), 0, s, a); break;
+      case ALPX_F32_PLANES:
+        hipLaunchKernelGGL(recurrent_chunk_prep_kernel<planes_t>, grid, dim3(256), 0, s, a);
+        break;
       default: hipLaunchKernelGGL(recurrent_chunk_prep_kernel<bf16_t>, grid, dim3(256), 0, s, a); break;
     }
   }
   int rc = check_launch("alpx_recurrent_prefill_prep");
-  if (rc != ALPX_OK || conv_kernel <= 1) return rc;
+  if (rc != ALPX_OK || conv_kernel <= 1 || tiled) return rc;
   const int C = 2 * key_heads * key_dim + value_heads * value_dim;
   hipLaunchKernelGGL(conv_history_advance, dim3((unsigned)((C + 255) / 256)), dim3(256), 0, s,
                      conv_history, current, tokens, conv_kernel, C);

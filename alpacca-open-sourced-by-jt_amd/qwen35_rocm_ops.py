@@ -1303,10 +1303,17 @@ class Qwen35RocmOps:
         mfma = key_width in (64, 128, 256) and value_width % 16 == 0
         qkv_dtype = (torch.bfloat16 if mfma and operand_dtype == torch.bfloat16
                      else torch.float32)
+        # fp32 q / k reach the chunked kernels split into their bf16 planes
+        # (the same bits, split once here rather than in every block)
+        planes = (qkv_dtype == torch.float32 and state.data_ptr() % 16 == 0
+                  and _lib.lib().alpx_gdn_chunk_uses_mfma(
+                      _lib.F32_PLANES, tokens, key_heads, value_heads, key_width,
+                      value_width) == 1)
         q, k, v, beta, g = _ops.recurrent_prefill_prep(
             mixed, weights, history[batch_index] if kernel > 1 else None, beta_logits,
             alpha_logits, dt_bias, ssm_a, key_heads=key_heads, key_dim=key_width,
-            value_heads=value_heads, value_dim=value_width, eps=eps, qkv_dtype=qkv_dtype)
+            value_heads=value_heads, value_dim=value_width, eps=eps, qkv_dtype=qkv_dtype,
+            planes=planes)
         seq_state = state[batch_index:batch_index + 1]
         attended = _ops.gdn_chunk(seq_state, q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0),
                                   beta.unsqueeze(0), g.unsqueeze(0), out_dtype=torch.float32)

@@ -38,6 +38,17 @@ extern "C" {
  * qwen35_rocm_ops.py:153-158; fp16/bf16 are this library's extension). */
 enum alpx_dtype { ALPX_F32 = 0, ALPX_F16 = 1, ALPX_BF16 = 2 };
 
+/* float32 q and k as three bf16 planes, p0 = bf16(x), p1 = bf16(x - p0),
+ * p2 = bf16(x - p0 - p1), which hold any float32 value exactly, in the order
+ * the chunked GDN kernels load them: [batch, key head, 16-token tile,
+ * key_dim / 32, plane, 64, 8], where lane 16 i + r holds channels 8 i ..
+ * 8 i + 7 of the k step of token r of the tile; the last tile's rows past
+ * the last token are zeros.  v stays float32.  What
+ * alpx_recurrent_prefill_prep writes and alpx_gdn_chunk_prefill reads in
+ * place of ALPX_F32 (the same result, without splitting every row once per
+ * block that uses it); no other entry point takes it. */
+enum { ALPX_F32_PLANES = 3 };
+
 enum alpx_status {
   ALPX_OK = 0,
   ALPX_EINVAL = -1,       /* contract violation: maps to ValueError/TypeError */
@@ -362,8 +373,9 @@ int alpx_gdn_chunk_uses_mfma(int dtype, int tokens, int key_heads, int value_hea
  * chunked MFMA kernels (workspace of alpx_gdn_chunk_workspace_bytes
  * needed; alpx_gdn_chunk_uses_mfma tells); fp32 inputs enter those
  * products as hi + lo bf16 pairs, so their result stays within fp32
- * accuracy (1e-4) of the token-sequential recurrence.  Anything else runs
- * the step kernel token by token (workspace unused).
+ * accuracy (1e-4) of the token-sequential recurrence (ALPX_F32_PLANES: q
+ * and k already split; the same result).  Anything else runs the step
+ * kernel token by token (workspace unused; ALPX_F32_PLANES is refused).
  */
 int alpx_gdn_chunk_prefill(float* state, const void* q, const void* k, const void* v,
                            const float* beta, const float* log_decay, void* out, void* workspace,
@@ -629,7 +641,9 @@ int alpx_attention_layer_prefill_paged(const void* query_gate, const void* key,
  * per-token chain of qwen35_numpy.py:63-131 that the reference's
  * token-sequential prefill runs, qwen35_runtime.py:777-810); the chunk
  * then runs alpx_gdn_chunk_prefill and the gated alpx_row_norm.  All
- * inputs fp32.  Two launches. */
+ * inputs fp32.  out_dtype may be ALPX_F32_PLANES (v_out then fp32).  One
+ * launch for kernels of up to 4 taps, head dims that are multiples of 4 and
+ * 16-byte aligned rows, else two. */
 int alpx_recurrent_prefill_prep(const float* current, const float* conv_weight,
                                 int64_t weight_tap_stride, int64_t weight_channel_stride,
                                 float* conv_history, int conv_kernel, const float* beta_logits,

@@ -305,6 +305,42 @@ def test_recurrent_prefill_prep_four_taps_equal_dims(gpu, tokens, hk, hv, d, lay
     assert np.array_equal(H.cpu().numpy(), hist[0].astype(np.float32))
 
 
+@pytest.mark.parametrize("tokens,kernel,hk,hv,dk,dv", [
+    (70, 4, 2, 4, 128, 128), (64, 3, 2, 4, 64, 32), (33, 4, 1, 2, 256, 16), (2, 4, 2, 2, 128, 64),
+    (1, 1, 1, 2, 64, 16), (90, 6, 2, 4, 128, 32), (130, 2, 3, 3, 64, 48)])
+def test_recurrent_prefill_prep_planes(gpu, tokens, kernel, hk, hv, dk, dv):
+    """q and k as bf16 planes (the tiled and, with 6 taps, the per-wave prep):
+    the planes add up to the fp32 values bit for bit, rows past the last
+    token are zeros, v / beta / decay / history are those of the fp32 form,
+    and the chunked GDN gives the fp32 form's bits from them -- token counts
+    that end inside a 16-token tile, chunks with idle waves, every head dim."""
+    import torch
+    P = _mod("_ops")
+    rng = np.random.default_rng(tokens + dk)
+    x = _rec_inputs(rng, tokens, hk, hv, dk, dv, kernel)
+    res = []
+    for planes in (False, True):
+        H = _f32(torch, x["hist"], gpu) if kernel > 1 else None
+        S = _f32(torch, x["s0"], gpu)[None].contiguous()
+        q, k, v, beta, g = P.recurrent_prefill_prep(
+            _f32(torch, x["mixed"], gpu), _f32(torch, x["w"], gpu), H, _f32(torch, x["bl"], gpu),
+            _f32(torch, x["al"], gpu), _f32(torch, x["dt"], gpu), _f32(torch, x["ssm"], gpu),
+            key_heads=hk, key_dim=dk, value_heads=hv, value_dim=dv, eps=1e-6,
+            qkv_dtype=torch.float32, planes=planes)
+        o = P.gdn_chunk(S, q[None], k[None], v[None], beta[None], g[None],
+                        out_dtype=torch.float32)
+        res.append((q, k, v, beta, g, o, S) + ((H,) if H is not None else ()))
+    torch.cuda.synchronize()
+    for rows, frag in zip(res[0][:2], res[1][:2]):
+        # [Hk, tile, ks, plane, 4 quads x 16 rows, 8] -> [tile, row, Hk, ks, quad, 8]
+        f = frag.float().reshape(hk, -1, dk // 32, 3, 4, 16, 8)
+        f = (f[:, :, :, 0] + f[:, :, :, 1] + f[:, :, :, 2]).permute(1, 4, 0, 2, 3, 5)
+        f = f.reshape(-1, hk, dk)
+        assert torch.equal(f[:tokens], rows) and not f[tokens:].any()
+    for a, b in zip(res[0][2:], res[1][2:]):
+        assert torch.equal(a, b)
+
+
 def _recurrent_prefill_vs_chain(ops, gpu, tokens, hk, hv, dk, dv, operand_dtype, seed=None,
                                 kernel=4):
     # the chunk (prep -> chunked GDN -> gated norm) of the second sequence of
