@@ -20,8 +20,15 @@
 //    O^T = V^T P^T, so the probabilities never leave the registers the
 //    score MFMA wrote them to.  The softmax max is a 2-step cross-lane
 //    (xor 16, xor 32) reduction.
-//  * everything else (fp32, odd head dims, unaligned caches):
+//  * fp32, the same head dims (decode_split_f32): the same structure on
+//    v_mfma_f32_16x16x4_f32.
+//  * everything else (odd head dims, unaligned caches):
 //    decode_split_generic, one wavefront per block, VALU dot products.
+//
+// Short caches, and batches that fill the device with one block a
+// (sequence, kv head), run one launch (decode_direct, one_launch): the same
+// kernels with up to 16 wavefronts, whose block has every row of its
+// sequence and writes the output.
 //
 // Pass 2 (combine): per (sequence, query head, 64 output columns), merge the
 // block partials with weights 2^(m_s - M), divide by the merged sum, apply
@@ -48,9 +55,14 @@ constexpr float kDecodeRescale = 8.0f;
 constexpr int kAuxNontemporal = 2;
 constexpr int kWaves = 4;   // wavefronts (= slots) per block (MFMA path)
 constexpr int kGenericTile = 64;
+constexpr int kMaxGridZ = 65535;
 constexpr int kMaxSlots = 2048;
 // Wave tile rows of the fp32 MFMA split kernel.
 constexpr int f32_tile_rows(int d) { return d == 64 ? 32 : 16; }
+// Wavefronts of a block that attends a whole sequence alone (one launch):
+// as many as leave the LDS of a CU its tiles (head_dim 128 fills it with 8;
+// fp32 at 64 takes 16 of 16 rows, 12.4 -> 11.7 us at 512 rows).
+constexpr int direct_waves(int d, int es) { return d == 256 ? 4 : (es == 4 && d == 64 ? 16 : 8); }
 constexpr int kMaxResident = 8192;  // upper bound on resident blocks any plan assumes
 
 
@@ -281,6 +293,63 @@ constexpr int merge_lds_bytes() {
   return 4 * ((kWaves - 1) * (D / 16) * 64 * 4 + 2 * (kWaves - 1) * 64);
 }
 
+// End of a block that has all rows of its sequence: the NW waves' states
+// are merged through LDS, normalised, gated and stored by the whole block.
+// h0, heads: the block's first query head and its live heads.
+template <int D, int NW>
+constexpr int direct_lds_bytes() {
+  return 4 * (NW * 16 * (D + 4) + 2 * NW * 16);
+}
+
+template <typename T, int D, int NW>
+__device__ __forceinline__ void write_out(const DecodeArgs& a, char* smem, f32x4 (&o)[D / 16],
+                                          float m, float l, int wave, int lane, bool head_ok,
+                                          int b, int h0, int heads) {
+  constexpr int kRow = D + 4;  // floats
+  const int hl = lane & 15;
+  const int quad = lane >> 4;
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  float* mo = (float*)smem;            // [NW][16][kRow]
+  float* mm = mo + NW * 16 * kRow;     // [NW][16]
+  float* ml = mm + NW * 16;
+  __syncthreads();
+  if (head_ok) {
+#pragma unroll
+    for (int mb = 0; mb < D / 16; ++mb)
+      *(f32x4*)(mo + (wave * 16 + hl) * kRow + 16 * mb + 4 * quad) = o[mb];
+    if (quad == 0) {
+      mm[wave * 16 + hl] = m;
+      ml[wave * 16 + hl] = l;
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < heads * D; i += 64 * NW) {
+    const int g = i / D;
+    const int d = i - g * D;
+    float M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, mm[w * 16 + g]);
+    float L = 0.f, A = 0.f;
+    if (M != -INFINITY) {
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float c = fast_exp2(mm[w * 16 + g] - M);
+        L += ml[w * 16 + g] * c;
+        A += mo[(w * 16 + g) * kRow + d] * c;
+      }
+    }
+    const int64_t bh = (int64_t)b * a.q_heads + h0 + g;
+    float r = L > 0.f ? A / L : 0.f;
+    if (a.gate != nullptr) r *= stable_sigmoid(to_f32(((const T*)a.gate)[bh * a.gate_stride + d]));
+    switch (a.out_dtype) {
+      case ALPX_F32: ((float*)a.out)[bh * D + d] = r; break;
+      case ALPX_F16: ((f16_t*)a.out)[bh * D + d] = from_f32<f16_t>(r); break;
+      default: ((bf16_t*)a.out)[bh * D + d] = from_f32<bf16_t>(r); break;
+    }
+  }
+}
+
 // ------------------------------------------------------------ MFMA split
 
 // One block = 4 wavefronts sharing one chunk of rows of one (sequence, kv
@@ -302,7 +371,10 @@ constexpr int merge_lds_bytes() {
 // way and put it and the value row into their staged tile in LDS, over
 // whatever their own loads fetched of that row; the one with head chunk 0
 // also writes both rows to the cache.
-template <typename T, int D, bool PAGED, bool PRO>
+//
+// DIRECT: the block has all rows of its sequence (one chunk) and writes the
+// output itself (write_out) instead of a partial.
+template <typename T, int D, bool PAGED, bool PRO, int NW, bool DIRECT>
 __device__ __forceinline__ void split_body(const DecodeArgs& a, const SplitPrologue* pp) {
   typedef typename Vec8<T>::type V8;
   typedef typename Vec4<T>::type V4;
@@ -310,11 +382,12 @@ __device__ __forceinline__ void split_body(const DecodeArgs& a, const SplitProlo
   constexpr int kUnits = D / 8;           // 16-byte units per row
   constexpr int kIters = kTile * kUnits / 64;
   constexpr int kTileElems = kTile * kStride;
-  constexpr int kTileBytes = 2 * kWaves * kTileElems * (int)sizeof(T);
-  constexpr int kLdsBytes = kTileBytes > merge_lds_bytes<D>() ? kTileBytes : merge_lds_bytes<D>();
+  constexpr int kTileBytes = 2 * NW * kTileElems * (int)sizeof(T);
+  constexpr int kMergeBytes = DIRECT ? direct_lds_bytes<D, NW>() : merge_lds_bytes<D>();
+  constexpr int kLdsBytes = kTileBytes > kMergeBytes ? kTileBytes : kMergeBytes;
   // PRO: 16 query rows and the new key and value rows (T), then one float
   // row per wave for the rotation partners.
-  constexpr int kProBytes = PRO ? (16 + 2) * D * (int)sizeof(T) + kWaves * D * 4 : 0;
+  constexpr int kProBytes = PRO ? (16 + 2) * D * (int)sizeof(T) + NW * D * 4 : 0;
   __shared__ __attribute__((aligned(16))) char smem[kLdsBytes + kProBytes];
 
   const int lane = threadIdx.x & 63;
@@ -382,7 +455,7 @@ __device__ __forceinline__ void split_body(const DecodeArgs& a, const SplitProlo
       }
     }
     // query heads hc * 16 + j of this kv group, one wave per head
-    for (int j = wave; j < 16; j += kWaves) {
+    for (int j = wave; j < 16; j += NW) {
       const int g = hc * 16 + j;
       if (g >= a.group) break;
       const T* src = (const T*)pp->qg + ((int64_t)b * a.q_heads + kvh * a.group + g) * (2 * D);
@@ -456,7 +529,7 @@ __device__ __forceinline__ void split_body(const DecodeArgs& a, const SplitProlo
   int p0 = start + kTile * wave;
   if (p0 < end) load_tile(p0);
   while (p0 < end) {
-    const int pn = p0 + kTile * kWaves;
+    const int pn = p0 + kTile * NW;
     // Stage K and V in LDS (row-major, padded rows), then prefetch the next tile.
 #pragma unroll
     for (int it = 0; it < kIters; ++it) {
@@ -536,19 +609,23 @@ __device__ __forceinline__ void split_body(const DecodeArgs& a, const SplitProlo
     p0 = pn;
   }
 
-  merge_waves<D>(a, smem, o, m, l, wave, lane, head_ok, b, h, slot);
+  if constexpr (DIRECT)
+    write_out<T, D, NW>(a, smem, o, m, l, wave, lane, head_ok, b, kvh * a.group + hc * 16,
+                        min(a.group - hc * 16, 16));
+  else
+    merge_waves<D>(a, smem, o, m, l, wave, lane, head_ok, b, h, slot);
 }
 
 template <typename T, int D, bool PAGED>
 __global__ void __launch_bounds__(256)
 decode_split_mfma(DecodeArgs a) {
-  split_body<T, D, PAGED, false>(a, nullptr);
+  split_body<T, D, PAGED, false, kWaves, false>(a, nullptr);
 }
 
 template <typename T, int D, bool PAGED>
 __global__ void __launch_bounds__(256)
 decode_split_mfma_pro(DecodeArgs a, SplitPrologue pp) {
-  split_body<T, D, PAGED, true>(a, &pp);
+  split_body<T, D, PAGED, true, kWaves, false>(a, &pp);
 }
 
 // fp32 caches: the same split structure on v_mfma_f32_16x16x4_f32 (fp32
@@ -560,16 +637,16 @@ decode_split_mfma_pro(DecodeArgs a, SplitPrologue pp) {
 //     4 quad + j] (one 16-byte LDS read per g) and Q[head hl][same d];
 //   O^T = V^T P^T, k-step (blk, i): lane supplies P[16 blk + 4 quad + i]
 //     [head hl] (its own score slot) and V[that row][16 mb + hl].
-template <int D, int R, bool PAGED>
-__global__ void __launch_bounds__(256)
-decode_split_f32(DecodeArgs a) {
+template <int D, int R, bool PAGED, int NW, bool DIRECT>
+__device__ __forceinline__ void split_f32_body(const DecodeArgs& a) {
   constexpr int kStride = D + 4;  // floats: rows 4 apart sit 16 banks apart
   constexpr int kUnits = D / 4;   // 16-byte units per row
   constexpr int kIters = R * kUnits / 64;
   constexpr int kTileElems = R * kStride;
   constexpr int NB = R / 16;
-  constexpr int kTileBytes = 2 * kWaves * kTileElems * 4;
-  constexpr int kLdsBytes = kTileBytes > merge_lds_bytes<D>() ? kTileBytes : merge_lds_bytes<D>();
+  constexpr int kTileBytes = 2 * NW * kTileElems * 4;
+  constexpr int kMergeBytes = DIRECT ? direct_lds_bytes<D, NW>() : merge_lds_bytes<D>();
+  constexpr int kLdsBytes = kTileBytes > kMergeBytes ? kTileBytes : kMergeBytes;
   static_assert(kIters >= 1 && R * kUnits % 64 == 0, "tile must split evenly over a wave");
   __shared__ __attribute__((aligned(16))) char smem[kLdsBytes];
 
@@ -631,7 +708,7 @@ decode_split_f32(DecodeArgs a) {
   int p0 = start + R * wave;
   if (p0 < end) load_tile(p0);
   while (p0 < end) {
-    const int pn = p0 + R * kWaves;
+    const int pn = p0 + R * NW;
 #pragma unroll
     for (int it = 0; it < kIters; ++it) {
       const int u = it * 64 + lane;
@@ -693,8 +770,36 @@ decode_split_f32(DecodeArgs a) {
     wave_sync_lds();
     p0 = pn;
   }
-  merge_waves<D>(a, smem, o, m, l, wave, lane, head_ok, b, h, slot);
+  if constexpr (DIRECT)
+    write_out<float, D, NW>(a, smem, o, m, l, wave, lane, head_ok, b, kvh * a.group + hc * 16,
+                        min(a.group - hc * 16, 16));
+  else
+    merge_waves<D>(a, smem, o, m, l, wave, lane, head_ok, b, h, slot);
 }
+
+template <int D, int R, bool PAGED>
+__global__ void __launch_bounds__(256)
+decode_split_f32(DecodeArgs a) {
+  split_f32_body<D, R, PAGED, kWaves, false>(a);
+}
+
+// ------------------------------------------------------------ one launch
+
+template <typename T, int D, bool PAGED>
+__global__ void __launch_bounds__(64 * direct_waves(D, sizeof(T)))
+decode_direct(DecodeArgs a) {
+  if constexpr (sizeof(T) == 4)
+    split_f32_body<D, 16, PAGED, direct_waves(D, 4), true>(a);
+  else
+    split_body<T, D, PAGED, false, direct_waves(D, sizeof(T)), true>(a, nullptr);
+}
+
+template <typename T, int D, bool PAGED>
+__global__ void __launch_bounds__(64 * direct_waves(D, sizeof(T)))
+decode_direct_pro(DecodeArgs a, SplitPrologue pp) {
+  split_body<T, D, PAGED, true, direct_waves(D, sizeof(T)), true>(a, &pp);
+}
+
 
 // ------------------------------------------------------------ generic split
 
@@ -1063,6 +1168,67 @@ const void* split_kernel(bool mfma, bool paged, int D) {
   return (const void*)decode_split_generic<T>;
 }
 
+// Kernel of a one-launch decode, which attends each sequence by one block.
+template <typename T, bool PRO, bool PAGED>
+const void* direct_kernel_of(int D) {
+  if constexpr (PRO && sizeof(T) == 4) {
+    return nullptr;
+  } else if constexpr (PRO) {
+    return D == 64 ? (const void*)decode_direct_pro<T, 64, PAGED>
+                   : (D == 128 ? (const void*)decode_direct_pro<T, 128, PAGED>
+                               : (const void*)decode_direct_pro<T, 256, PAGED>);
+  } else {
+    return D == 64 ? (const void*)decode_direct<T, 64, PAGED>
+                   : (D == 128 ? (const void*)decode_direct<T, 128, PAGED>
+                               : (const void*)decode_direct<T, 256, PAGED>);
+  }
+}
+
+template <typename T>
+const void* direct_kernel(bool pro, bool paged, int D) {
+  if (pro) return paged ? direct_kernel_of<T, true, true>(D) : direct_kernel_of<T, true, false>(D);
+  return paged ? direct_kernel_of<T, false, true>(D) : direct_kernel_of<T, false, false>(D);
+}
+
+// Whether one block a (sequence, kv head, 16 query heads) attends all rows
+// and writes the output, in place of the split and combine launches.  The
+// second launch costs about 3.5 us of a short step (two launches never took
+// less than 7-8 us, one 4-5 us), and with the device full of sequences the
+// partials and the many short blocks cost more than uneven CUs do; a block
+// alone streams a step of 256 rows (128 at head_dim 256) in 2-2.6 us.
+// Measured (bf16, us, two launches / one; the rows are what the cache
+// holds, graph replays over three buffers):
+//   few blocks: 8 of head_dim 128: 256 rows 8.5 / 5.8, 384 8.8 / 7.7, 512
+//     8.5 / 9.2; 8 of 64: 512 7.6 / 5.5, 768 6.8 / 7.1; 2 of 256: 128 rows
+//     10.4 / 8.1, 256 10.9 / 11.3
+//   128 blocks, half the CUs: 1024 rows 18.5 / 16.8 at 128, 13.1 / 11.8 at
+//     64, 32.1 / 28.7 at 256; 2048 rows even
+//   256 blocks of 128: 2048 rows 55.1 / 45.9; 512: 89.1 / 81.4; 1024:
+//     185.9 / 168.3; but 320, which leave 3/8 of two rounds of CUs idle:
+//     1024 rows 34.4 / 36.4.
+// One head a block leaves so few partials that the two launches stay ahead
+// in the cases above at the edge: 128 blocks of head_dim 256, 1024 rows
+// 31.2 / 32.6; 2048 of 128, 256 rows 53.9 / 61.0 (four heads 65.3 / 61.9).
+// Device lengths (`ragged`) take it only where a block alone is the faster
+// at any number of them: the balanced plan's time follows the total, the
+// one launch's the longest.  fp32 steps are bound by the MFMA rate of a
+// block (16 columns for a group of 4): 8 blocks of head_dim 64, 256 rows
+// 8.7 / 7.4, 512 9.0 / 11.1; of 128, 128 rows 9.4 / 7.7, 256 9.4 / 11.4; 2
+// of 256, 64 rows 12.3 / 9.8, 128 12.5 / 14.0; 2048 blocks lose at any
+// length (31.9 / 38.4 at 64 rows).
+bool one_launch(int D, int dtype, int group, int blocks, int length, bool ragged) {
+  const int cus = multiprocessor_count();
+  if (dtype == ALPX_F32)
+    return blocks <= 2 * cus && length <= (D == 64 ? 256 : (D == 128 ? 128 : 64));
+  if (!ragged && group < 4 && blocks > 2 * cus) return false;
+  if (length <= (D == 64 ? 512 : (D == 128 ? 384 : 128))) return true;
+  if (ragged || length > 2048) return false;
+  const int rounds = (blocks + cus - 1) / cus;
+  const float fill = (float)blocks / ((float)rounds * (float)cus);
+  if (length > 1024) return fill >= 0.9f;
+  return fill >= (rounds > 1 ? 0.8f : (group < 4 ? 0.6f : 0.5f));
+}
+
 template <typename T, int NW, int G>
 void launch_combine_nw(int out_dtype, const DecodeArgs& a, hipStream_t s) {
   const dim3 grid(a.batch * a.q_heads, (a.value_dim + 63) / 64), block(64 * NW);
@@ -1091,10 +1257,10 @@ int launch_combine(int out_dtype, const DecodeArgs& a, hipStream_t s) {
   return check_launch("decode_combine");
 }
 
-int launch_split(const void* kernel, bool mfma, const DecodeArgs& a, const SplitPrologue* pro,
+int launch_split(const void* kernel, int threads, const DecodeArgs& a, const SplitPrologue* pro,
                  dim3 grid, hipStream_t s) {
   void* args[] = {(void*)&a, (void*)pro};
-  hipError_t err = hipLaunchKernel(kernel, grid, dim3(mfma ? 256 : 64), args, 0, s);
+  hipError_t err = hipLaunchKernel(kernel, grid, dim3(threads), args, 0, s);
   if (err != hipSuccess)
     return fail(ALPX_EHIP, "decode split launch failed: %s", hipGetErrorString(err));
   return check_launch("decode_split");
@@ -1210,6 +1376,18 @@ int run_decode(DecodeArgs a, int dtype, int out_dtype, void* workspace, size_t w
                 "%s: this call needs %zu bytes of split partials, more than the %zu-byte static "
                 "scratch (call the entry point that takes a workspace)",
                 fixed_scratch, partial_bytes(n, a.value_dim), workspace_bytes);
+  if (mfma && a.causal_pos0 < 0 && a.batch <= kMaxGridZ &&
+      one_launch(D, dtype, a.group, a.batch * rows_y, a.length, a.seq_lens != nullptr)) {
+    const void* direct = dtype == ALPX_F32   ? direct_kernel<float>(pro != nullptr, paged, D)
+                         : dtype == ALPX_F16 ? direct_kernel<f16_t>(pro != nullptr, paged, D)
+                                             : direct_kernel<bf16_t>(pro != nullptr, paged, D);
+    a.balanced = a.skew = 0;
+    a.nsplit = 1;
+    a.chunk = a.length;
+    a.out_dtype = out_dtype;
+    TimedRegion timed(split_timer, s);
+    return launch_split(direct, 64 * direct_waves(D, (int)es), a, pro, dim3(1, rows_y, a.batch), s);
+  }
   char* ws = (char*)workspace;
   a.part_m = (float*)ws;
   a.part_l = (float*)(ws + align256(n * sizeof(float)));
@@ -1217,7 +1395,7 @@ int run_decode(DecodeArgs a, int dtype, int out_dtype, void* workspace, size_t w
   int rc;
   {
     TimedRegion timed(split_timer, s);
-    rc = launch_split(kernel, mfma, a, pro, grid, s);
+    rc = launch_split(kernel, mfma ? 64 * kWaves : 64, a, pro, grid, s);
   }
   if (rc != ALPX_OK) return rc;
   TimedRegion timed(combine_timer, s);

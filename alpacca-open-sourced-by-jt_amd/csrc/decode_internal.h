@@ -59,6 +59,7 @@ struct DecodeArgs {
   int items_target;  // blocks per grid row the chunk size is cut for
   int items_max;     // grid x: at least the item count
   int unit;          // rows per block step of the split kernel
+  int out_dtype;     // one-launch decode: type of `out`
 };
 
 // The Qwen3.5 attention prologue fused into the split launch: one new token

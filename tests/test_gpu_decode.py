@@ -278,6 +278,59 @@ def test_decode_split_plans_against_oracle(gpu, ops, B, length, hq, hkv, d, dtyp
     assert err <= TOL[dtype], err
 
 
+@pytest.mark.parametrize("hq,hkv,d,length,dtype,kind", [
+    (4, 1, 64, 1, "bf16", "gate"), (8, 2, 64, 31, "f16", "paged"),
+    (34, 2, 64, 255, "bf16", "ragged"),       # 17 heads a group: two column blocks
+    (8, 2, 64, 512, "f16", "ragged"), (8, 2, 64, 513, "f16", "ragged"),
+    (32, 8, 128, 33, "bf16", "ragged"), (8, 8, 128, 257, "f16", "gate"),
+    (8, 2, 128, 384, "bf16", "paged"), (8, 2, 128, 385, "bf16", "paged"),
+    (16, 2, 256, 127, "bf16", "gate"), (40, 2, 256, 128, "f16", "paged"),
+    (16, 2, 256, 129, "bf16", "ragged"),
+    (8, 2, 64, 15, "f32", "gate"), (34, 2, 64, 256, "f32", "ragged"),
+    (8, 2, 64, 257, "f32", "paged"), (8, 2, 128, 128, "f32", "paged"),
+    (8, 2, 128, 129, "f32", "ragged"), (4, 2, 256, 64, "f32", "gate"),
+    (4, 2, 256, 65, "f32", "ragged")])
+def test_decode_one_launch_edges(gpu, ops, hq, hkv, d, length, dtype, kind):
+    """Caches up to and just past the length that one block a (sequence, kv
+    head) attends alone: wave tiles with a remainder, more waves than tiles,
+    empty sequences, the gate and pages.  Tolerances as everywhere here: the
+    products and sums are those of the split kernels."""
+    import torch
+    rng = np.random.default_rng(hq * 1000 + d + length)
+    B = 3
+    q = I.round_to(rng.standard_normal((B, hq, d)), dtype)
+    K = I.round_to(rng.standard_normal((length, B, hkv, d)), dtype)
+    V = I.round_to(rng.standard_normal((length, B, hkv, d)), dtype)
+    gate = I.round_to(rng.standard_normal((B, hq, d)), dtype) if kind == "gate" else None
+    lens = [length, 0, (length + 1) // 2] if kind == "ragged" else [length] * B
+    seq = torch.tensor(lens, dtype=torch.int32, device=gpu) if kind == "ragged" else None
+    if kind == "paged":
+        page = 32
+        n = -(-length // page)
+        table = rng.permutation(B * n + 2)[:B * n].reshape(B, n)
+        pages = np.zeros((2, B * n + 2, page, hkv, d), np.float32)
+        for i, rows in enumerate((K, V)):
+            for b in range(B):
+                for r in range(length):
+                    pages[i, table[b, r // page], r % page] = rows[r, b]
+        out = ops.paged_online_attention(
+            _dev(torch, q, dtype, gpu), _dev(torch, pages[0], dtype, gpu),
+            _dev(torch, pages[1], dtype, gpu), torch.from_numpy(table.astype(np.int32)).to(gpu),
+            length=length, out_dtype=torch.float32)
+    else:
+        out = ops.online_attention(
+            _dev(torch, q, dtype, gpu), _dev(torch, K, dtype, gpu), _dev(torch, V, dtype, gpu),
+            length=length, seq_lens=seq, out_dtype=torch.float32,
+            gate=None if gate is None else _dev(torch, gate, dtype, gpu))
+    for b, n in enumerate(lens):
+        ref = np.zeros((hq, d)) if n == 0 else A.online_attention(
+            q[b:b + 1], K[:, b:b + 1], V[:, b:b + 1], n)[0]
+        if gate is not None:
+            ref = ref / (1.0 + np.exp(-gate[b].astype(np.float64)))
+        err = np.abs(out[b].cpu().numpy() - ref).max()
+        assert err <= TOL[dtype], (b, err)
+
+
 def test_decode_repeatable_across_plans(gpu, ops):
     import torch
     rng = np.random.default_rng(11)
