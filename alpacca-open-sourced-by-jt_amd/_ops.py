@@ -147,7 +147,11 @@ def _split_workspace(L, device, *sizes):
     """Workspace of its own for an MFMA prefill that cuts its key ranges over
     several blocks (None where the chunk runs unsplit): from torch's
     stream-ordered allocator, so that calls on different streams share
-    nothing.  ``sizes``: the arguments of alpx_prefill_split_bytes."""
+    nothing.  ``sizes``: the arguments of alpx_prefill_split_bytes, which is
+    0 up to 480 cache rows (7 key tiles of 64, 15 of 32): the shortest
+    calls, bound by their host time, don't ask."""
+    if sizes[1] <= 480:
+        return None
     nbytes = L.alpx_prefill_split_bytes(*sizes)
     return _torch().empty(nbytes, dtype=_torch().uint8, device=device) if nbytes else None
 

@@ -453,3 +453,15 @@ def test_random_attention_batch_seam_against_oracle(gpu, c):
     assert err <= tol, (c["id"], err)
     if c["t_q"] > 1:
         assert seam.attention_batch(q, K, V, pos[::-1].copy(), c["group"], inv) is None
+
+
+def test_prefill_up_to_480_rows_is_not_split(gpu):
+    """The host asks for no split workspace up to 480 cache rows."""
+    L = importlib.import_module("alpacca-open-sourced-by-jt_amd._lib").lib()
+    for kv in (1, 63, 64, 65, 257, 448, 449, 480):
+        for tokens in (1, 2, 9, 16, 40, 200, kv):
+            for hq, hkv in ((32, 8), (16, 2), (8, 8), (4, 1), (1, 1)):
+                for d in (64, 128, 256):
+                    for window in (0, 100):
+                        assert tokens > kv or L.alpx_prefill_split_bytes(
+                            tokens, kv, hq, hkv, d, kv - tokens, window, 0) == 0
