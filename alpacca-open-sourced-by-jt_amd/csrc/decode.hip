@@ -38,6 +38,7 @@
 // and invalidate the XCD L2 in every block.)
 #include <math.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "alpx_common.h"
@@ -97,7 +98,8 @@ __device__ __forceinline__ int seq_lo(const DecodeArgs& a, int b, int hi) {
 // of the lengths, so the step time follows the total row count, not the
 // longest sequence.  Since sum_b ceil(len_b / C) <= total / C + batch <=
 // items_target + batch, the grid (items_max = items_target + batch) holds
-// every item; blocks past the last item exit.  The functions below are
+// every item; blocks past the last item exit.  Up to one_rows rows in all C
+// is cut for items_one blocks instead, so that the items run in one round.  The functions below are
 // wave-collective (every lane of the calling wave active) and every wave
 // that calls them gets the same result.
 
@@ -129,7 +131,10 @@ __device__ __forceinline__ int balanced_chunk(const DecodeArgs& a, int lane, int
   // 32-bit divisions where the row total allows (the 64-bit ones are long
   // instruction sequences on the path to every block's first tile loads)
   int64_t c;
-  if (total <= 0x7fffffff - a.items_target) {
+  if (total <= a.one_rows) {
+    const unsigned q = ((unsigned)total + (unsigned)a.items_one - 1u) / (unsigned)a.items_one;
+    c = (q + (unsigned)a.unit - 1u) / (unsigned)a.unit * (unsigned)a.unit;
+  } else if (total <= 0x7fffffff - a.items_target) {
     const unsigned q = ((unsigned)total + (unsigned)a.items_target - 1u) / (unsigned)a.items_target;
     c = (q + (unsigned)a.unit - 1u) / (unsigned)a.unit * (unsigned)a.unit;
   } else {
@@ -374,7 +379,14 @@ __device__ __forceinline__ void write_out(const DecodeArgs& a, char* smem, f32x4
 //
 // DIRECT: the block has all rows of its sequence (one chunk) and writes the
 // output itself (write_out) instead of a partial.
-template <typename T, int D, bool PAGED, bool PRO, int NW, bool DIRECT>
+//
+// TWO: P enters its product in two parts, rounded and the rest.  P's
+// rounding is the error of the result, and where a wave has one tile its
+// largest P is the exact 1 (bf16, rms of the result 1.2e-3 with one tile a
+// wave, 1.5e-3 with two to eight, 2e-6 in two parts): the kernels that give
+// a wave several tiles where shorter chunks gave it one take two parts.  It
+// costs 0.2-0.3 us of a 10 us step, also behind a branch.
+template <typename T, int D, bool PAGED, bool PRO, int NW, bool DIRECT, bool TWO>
 __device__ __forceinline__ void split_body(const DecodeArgs& a, const SplitPrologue* pp) {
   typedef typename Vec8<T>::type V8;
   typedef typename Vec4<T>::type V4;
@@ -581,12 +593,14 @@ __device__ __forceinline__ void split_body(const DecodeArgs& a, const SplitProlo
     const float mn = grow ? mx : m;
     const float alpha = grow ? fast_exp2(m - mn) : 1.f;
     V8 pv;
+    [[maybe_unused]] V8 pr;
     float ps = 0.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const float p = fast_exp2(sv[j] - mn);
       ps += p;
       pv[j] = from_f32<T>(p);
+      if constexpr (TWO) pr[j] = from_f32<T>(p - to_f32(pv[j]));
     }
     l = l * alpha + ps;
     m = mn;
@@ -603,6 +617,7 @@ __device__ __forceinline__ void split_body(const DecodeArgs& a, const SplitProlo
       const V4 lo = lds_read_tr4(ldsv + tr_row * kStride + 16 * mb + tr_col);
       const V4 hi = lds_read_tr4(ldsv + (16 + tr_row) * kStride + 16 * mb + tr_col);
       const V8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      if constexpr (TWO) o[mb] = mfma16x16x32(va, pr, o[mb]);
       o[mb] = mfma16x16x32(va, pv, o[mb]);
     }
     wave_sync_lds();
@@ -616,16 +631,16 @@ __device__ __forceinline__ void split_body(const DecodeArgs& a, const SplitProlo
     merge_waves<D>(a, smem, o, m, l, wave, lane, head_ok, b, h, slot);
 }
 
-template <typename T, int D, bool PAGED>
+template <typename T, int D, bool PAGED, bool TWO = false>
 __global__ void __launch_bounds__(256)
 decode_split_mfma(DecodeArgs a) {
-  split_body<T, D, PAGED, false, kWaves, false>(a, nullptr);
+  split_body<T, D, PAGED, false, kWaves, false, TWO>(a, nullptr);
 }
 
-template <typename T, int D, bool PAGED>
+template <typename T, int D, bool PAGED, bool TWO = false>
 __global__ void __launch_bounds__(256)
 decode_split_mfma_pro(DecodeArgs a, SplitPrologue pp) {
-  split_body<T, D, PAGED, true, kWaves, false>(a, &pp);
+  split_body<T, D, PAGED, true, kWaves, false, TWO>(a, &pp);
 }
 
 // fp32 caches: the same split structure on v_mfma_f32_16x16x4_f32 (fp32
@@ -791,13 +806,13 @@ decode_direct(DecodeArgs a) {
   if constexpr (sizeof(T) == 4)
     split_f32_body<D, 16, PAGED, direct_waves(D, 4), true>(a);
   else
-    split_body<T, D, PAGED, false, direct_waves(D, sizeof(T)), true>(a, nullptr);
+    split_body<T, D, PAGED, false, direct_waves(D, sizeof(T)), true, true>(a, nullptr);
 }
 
 template <typename T, int D, bool PAGED>
 __global__ void __launch_bounds__(64 * direct_waves(D, sizeof(T)))
 decode_direct_pro(DecodeArgs a, SplitPrologue pp) {
-  split_body<T, D, PAGED, true, direct_waves(D, sizeof(T)), true>(a, &pp);
+  split_body<T, D, PAGED, true, direct_waves(D, sizeof(T)), true, true>(a, &pp);
 }
 
 
@@ -1109,6 +1124,25 @@ constexpr int kMaxItemsPerRow = 256;
 #define ALPX_BALANCED_SUB 0
 #endif
 
+// One round of longer chunks (items_one = resident blocks per grid row -
+// batch, so that no item is left for a second round) while a chunk stays at
+// most this many block steps: two and a half rounds of short totals are
+// blocks of one step, which pay a start and a merge each and fill the last
+// round badly.  Measured (bf16, split + combine, us, 5/2 rounds / one): with
+// two blocks a CU (head_dim 128, 32/8 heads) 18k rows of 8 sequences 25.6 /
+// 22.9, 9k of 16 19.6 / 17.9, but 24.6k of 16 (512-row chunks) 26.9 / 27.8;
+// with one (head_dim 256, 16/2 heads) 36k rows of 4 32.6 / 25.4, 69k of 16
+// (8 steps) 38.7 / 34.8, 103k of 16 54.1 / 49.7.  With
+// four (head_dim 64) others hide a block's start: 24k rows of 16 18.1 /
+// 19.1, so they keep the short chunks.  A batch that takes over a third of
+// the round's blocks leaves it half empty (32 sequences of 24/4 heads of
+// 256, 26k rows: 36.8 / 42.6), and fp32 steps, bound by the MFMA rate, gain
+// from more blocks (7k rows of 16 at head_dim 128 26.5 / 31.6).  The host
+// knows only that a total is at most batch x length: at most one step a
+// block, or more than twice the rule's rows, launch the kernel without it.
+constexpr int kOneRoundUnits1 = 8;
+constexpr int kOneRoundUnits2 = 3;
+
 // Grid x of the balanced plan: the item count is at most items_target +
 // batch (see balanced_chunk) and at most batch * ceil(length / unit) (no
 // chunk is shorter than unit rows unless it ends its sequence).
@@ -1196,8 +1230,8 @@ const void* direct_kernel(bool pro, bool paged, int D) {
 // less than 7-8 us, one 4-5 us), and with the device full of sequences the
 // partials and the many short blocks cost more than uneven CUs do; a block
 // alone streams a step of 256 rows (128 at head_dim 256) in 2-2.6 us.
-// Measured (bf16, us, two launches / one; the rows are what the cache
-// holds, graph replays over three buffers):
+// Measured (bf16, us, two launches / one, graph replays over three buffers;
+// P's second part has since added 0.1-0.2 us to the one):
 //   few blocks: 8 of head_dim 128: 256 rows 8.5 / 5.8, 384 8.8 / 7.7, 512
 //     8.5 / 9.2; 8 of 64: 512 7.6 / 5.5, 768 6.8 / 7.1; 2 of 256: 128 rows
 //     10.4 / 8.1, 256 10.9 / 11.3
@@ -1227,6 +1261,22 @@ bool one_launch(int D, int dtype, int group, int blocks, int length, bool ragged
   const float fill = (float)blocks / ((float)rounds * (float)cus);
   if (length > 1024) return fill >= 0.9f;
   return fill >= (rounds > 1 ? 0.8f : (group < 4 ? 0.6f : 0.5f));
+}
+
+// The split kernel of a balanced plan that may run in one round (head_dim
+// 128 and 256; the others never leave room for it).
+template <typename T, bool PAGED>
+const void* one_round_kernel_of(int D, bool pro) {
+  if (D == 128)
+    return pro ? (const void*)decode_split_mfma_pro<T, 128, PAGED, true>
+               : (const void*)decode_split_mfma<T, 128, PAGED, true>;
+  return pro ? (const void*)decode_split_mfma_pro<T, 256, PAGED, true>
+             : (const void*)decode_split_mfma<T, 256, PAGED, true>;
+}
+
+template <typename T>
+const void* one_round_kernel(int D, bool pro, bool paged) {
+  return paged ? one_round_kernel_of<T, true>(D, pro) : one_round_kernel_of<T, false>(D, pro);
 }
 
 template <typename T, int NW, int G>
@@ -1347,6 +1397,18 @@ int run_decode(DecodeArgs a, int dtype, int out_dtype, void* workspace, size_t w
     target = target < 1 ? 1 : (target > kMaxItemsPerRow ? kMaxItemsPerRow : target);
     a.balanced = 1;
     a.items_target = target;
+    const int per_cu = resident / multiprocessor_count();
+    const int one_units = per_cu <= 1 ? kOneRoundUnits1 : (per_cu == 2 ? kOneRoundUnits2 : 0);
+    const int one = std::min(resident / rows_y - a.batch, target);
+    const int64_t most = (int64_t)a.batch * a.length;
+    a.one_rows = -1;
+    if (mfma && es == 2 && D >= 128 && a.batch <= resident / rows_y / 3 &&
+        most > (int64_t)one * unit && most <= 2 * (int64_t)one * one_units * unit) {
+      a.one_rows = one * one_units * unit;
+      kernel = dtype == ALPX_F16 ? one_round_kernel<f16_t>(D, pro != nullptr, paged)
+                                 : one_round_kernel<bf16_t>(D, pro != nullptr, paged);
+    }
+    a.items_one = one;
     a.items_max = balanced_items_max(a.batch, a.length, unit, target);
     a.unit = unit;
     a.nsplit = balanced_slots(a.length, unit, target);

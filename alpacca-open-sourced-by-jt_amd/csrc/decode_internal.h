@@ -57,6 +57,8 @@ struct DecodeArgs {
   // nsplit bounds the chunks of one sequence.
   int balanced;
   int items_target;  // blocks per grid row the chunk size is cut for
+  int items_one;     // the same, totals of at most one_rows rows
+  int one_rows;      // -1: none
   int items_max;     // grid x: at least the item count
   int unit;          // rows per block step of the split kernel
   int out_dtype;     // one-launch decode: type of `out`

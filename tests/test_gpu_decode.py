@@ -331,6 +331,33 @@ def test_decode_one_launch_edges(gpu, ops, hq, hkv, d, length, dtype, kind):
         assert err <= TOL[dtype], (b, err)
 
 
+@pytest.mark.parametrize("hq,hkv,d,dtype,lens", [
+    (32, 8, 128, "bf16", [3000, 1, 2200, 0]),        # one round of 128-row chunks
+    (32, 8, 128, "f16", [5000, 6000, 5800, 6300]),   # one round, 3 steps a chunk
+    (32, 8, 128, "f16", [5900, 6000, 5800, 6300]),   # past it: two and a half rounds
+    (16, 2, 256, "bf16", [14000, 15500, 90, 8000]),  # one round, 3 steps at head_dim 256
+    (4, 1, 128, "bf16", [20000, 129]),               # more blocks a row than the plan cuts for
+    (32, 8, 64, "f32", [2500, 3000, 77])])
+def test_decode_balanced_rounds(gpu, ops, hq, hkv, d, dtype, lens):
+    """Device lengths whose totals fall on both sides of the one-round rule:
+    every row once, against the oracle."""
+    import torch
+    rng = np.random.default_rng(sum(lens))
+    B, C = len(lens), max(lens)
+    q = I.round_to(rng.standard_normal((B, hq, d)), dtype)
+    K = I.round_to(rng.standard_normal((C, B, hkv, d), dtype=np.float32), dtype)
+    V = I.round_to(rng.standard_normal((C, B, hkv, d), dtype=np.float32), dtype)
+    seq = torch.tensor(lens, dtype=torch.int32, device=gpu)
+    out = ops.online_attention(_dev(torch, q, dtype, gpu), _dev(torch, K, dtype, gpu),
+                               _dev(torch, V, dtype, gpu), length=C, seq_lens=seq,
+                               out_dtype=torch.float32)
+    for b, n in enumerate(lens):
+        ref = np.zeros((hq, d)) if n == 0 else A.online_attention(
+            q[b:b + 1], K[:, b:b + 1], V[:, b:b + 1], n)[0]
+        err = np.abs(out[b].cpu().numpy() - ref).max()
+        assert err <= TOL[dtype], (b, err)
+
+
 def test_decode_repeatable_across_plans(gpu, ops):
     import torch
     rng = np.random.default_rng(11)
