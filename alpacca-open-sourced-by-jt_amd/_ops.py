@@ -802,7 +802,8 @@ def attention_layer_prefill(query_gate, key, value, q_norm, k_norm, key_cache, v
             _lib.check(rc)
             return out
     query = torch.empty((tokens, q_heads, dim), dtype=key_cache.dtype, device=dev)
-    rc = call(query, _lib.workspace(torch, dev, split) if split else None)
+    # its own, as in prefill_append: this form shares no workspace between streams
+    rc = call(query, torch.empty(split, dtype=torch.uint8, device=dev) if split else None)
     if rc == _lib.EINVAL:  # the split-K prefill (fp32, unaligned, >= 2 GiB) needs a workspace
         nbytes = L.alpx_prefill_workspace_bytes(tokens, q_heads, kv_heads, dim,
                                                 int(position) + tokens)

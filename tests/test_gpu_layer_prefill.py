@@ -170,6 +170,30 @@ def test_attention_layer_prefill_equals_prologue_then_gated_prefill(gpu, hq, hkv
         assert torch.equal(out_a, out_b), fused
 
 
+def test_attention_layer_prefill_query_buffer_form_shares_no_workspace(gpu, monkeypatch):
+    """The query-buffer form of a chunk whose key ranges are split takes its
+    partials from a buffer of its own, so that calls on two streams share
+    nothing."""
+    import torch
+    P, Lib = _mod("_ops"), _mod("_lib")
+    hq, hkv, d, prefix, tokens = 8, 2, 128, 2500, 21
+    assert Lib.lib().alpx_prefill_split_bytes(tokens, prefix + tokens, hq, hkv, d, prefix, 0, 0) > 0
+    g = torch.Generator(device=gpu).manual_seed(3)
+    r = lambda *s: torch.randn(*s, generator=g, device=gpu)  # noqa: E731
+    b = lambda *s: r(*s).to(torch.bfloat16)  # noqa: E731
+    kc, vc = b(prefix + tokens, 1, hkv, d), b(prefix + tokens, 1, hkv, d)
+    args = (b(tokens, hq, 2 * d), b(tokens, hkv, d), b(tokens, hkv, d), r(d), r(d), kc, vc)
+    kw = dict(batch_index=0, position=prefix, sections=(11, 11, 10, 0), frequency_base=1e6,
+              eps=1e-6)
+    fused = P.attention_layer_prefill(*args, fused_query=True, **kw)
+
+    def shared(*_):
+        raise AssertionError("the shared workspace was taken")
+
+    monkeypatch.setattr(Lib, "workspace", shared)
+    assert torch.equal(P.attention_layer_prefill(*args, fused_query=False, **kw), fused)
+
+
 def test_attention_layer_prefill_cache_of_2gib_or_more(gpu, ops):
     """A chunk over caches of 2 GiB per tensor (16 sequences x 131072 rows of
     2 x 256 bf16): the MFMA prefill's 32-bit row offsets do not reach, so
