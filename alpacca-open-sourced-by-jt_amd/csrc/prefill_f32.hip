@@ -24,7 +24,7 @@ constexpr int f32_tile_keys(int d) { return d == 256 ? 16 : 32; }
 // reads and the softmax fit beside the other waves' products (32/8 heads,
 // 1000 tokens on 4096 rows: 119 TFLOP/s at head_dim 64, 125 at 128, where
 // a library product reaches 153).  1000 tokens on no prefix at head_dim 64
-// take 50 us, the heaviest blocks' 32 tiles in series; the decode machinery
+// take 51 us, the heaviest blocks' 32 tiles in series; the decode machinery
 // (one token per "sequence", 4 of 16 MFMA columns live) took 243.  Two
 // wave groups per block, each on half of its keys, measured 46 there and
 // 27% slower at head_dim 128.
@@ -96,9 +96,9 @@ prefill_f32(PrefillArgs a) {
   const float* vg = (const float*)a.v + (int64_t)kvh * D;
   const uint32_t lbase = (uint32_t)(uintptr_t)(lds_void_t*)smem;
   auto load_tile = [&](const float* g, int64_t pos, const uint32_t (&ofs)[kIW], int t, int buf) {
-    const int k0 = lo + t * BK;  // rows at or past kv_tokens read as zero
+    const int k0 = lo + t * BK;  // rows no column sees (at or past hi) read as zero
     const i32x4 r = rsrc_words((uint64_t)(uintptr_t)(g + (int64_t)k0 * pos),
-                               (uint32_t)((int64_t)(a.kv_tokens - k0) * pos * 4));
+                               (uint32_t)((int64_t)(hi - k0) * pos * 4));
     const uint32_t lds0 = lbase + buf * kTileB + wave * kIW * 1024;
 #pragma unroll
     for (int i = 0; i < kIW; ++i) lds_dma16(r, lds0 + i * 1024, ofs[i]);
@@ -193,6 +193,36 @@ prefill_f32(PrefillArgs a) {
               const float va = *(const float*)(vt + vadr[y] + (16 * blk + i) * kRowB + 64 * mb);
               t[y] = mfma16x16x4(va, s[blk][i], t[y]);
             }
+        if (edge) {
+          // a row that one column sees and another does not: if it holds an
+          // infinity or a NaN, 0 times it must not reach the other, so each
+          // token's columns take the product over their own rows alone
+          bool bad = false;
+#pragma unroll
+          for (int y = 0; y < 4; ++y)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bad |= !(fabsf(t[y][i]) < INFINITY);
+          if (__ballot(bad) != 0) {
+#pragma unroll
+            for (int y = 0; y < 4; ++y)
+#pragma clang loop unroll(disable)
+              for (int wt = wt_first; wt <= wt_last; ++wt) {
+                f32x4 u = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int blk = 0; blk < NB; ++blk)
+#pragma unroll
+                  for (int i = 0; i < 4; ++i) {
+                    const int key = k0 + 16 * blk + 4 * quad + i;
+                    const bool seen =
+                        key <= rel0 + wt && (a.window <= 0 || key > rel0 + wt - a.window);
+                    const float va =
+                        *(const float*)(vt + vadr[y] + (16 * blk + i) * kRowB + 64 * mb);
+                    u = mfma16x16x4(seen ? va : 0.f, s[blk][i], u);
+                  }
+                if (tok == wt) t[y] = u;
+              }
+          }
+        }
 #pragma unroll
         for (int y = 0; y < 4; ++y) o[mb + y] += t[y];
       }

@@ -123,6 +123,7 @@ prefill_combine(PrefillArgs a) {
     for (int i = 0; i < MW; ++i) o[i] *= keep;
 #pragma unroll
     for (int u = 0; u < kGroup; ++u) {
+      if (s0 + u >= cnt) continue;  // the last piece again: 0 times its infinities is a NaN
       const float wt = st[u].x == -INFINITY ? 0.f : fast_exp2(st[u].x - mg);
       L += wt * st[u].y;
 #pragma unroll

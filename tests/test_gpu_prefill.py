@@ -251,6 +251,35 @@ def test_prefill_f32_matches_oracle_and_decode_machinery(gpu, override, tq, pref
         assert np.all(got[:-pos_off] == 0.0)
 
 
+@pytest.mark.parametrize("tq,prefix,hq,hkv,d,window", [
+    (300, 0, 16, 8, 64, 0), (203, 43, 24, 8, 128, 50), (250, 30, 8, 8, 256, 0),
+    (40, 1500, 32, 8, 64, 0)])
+def test_prefill_f32_unseen_rows_never_reach_a_row(gpu, tq, prefix, hq, hkv, d, window):
+    """float32: infinities and NaN in rows past the chunk, and in the last
+    token's own row, leave every row that does not see them as it is, bit
+    for bit, and a seen infinity stays one, also in the last piece of a
+    split.  Sizes that prefill_f32 takes: whole and split key ranges, several
+    tokens in a wave, a window."""
+    import torch
+    P = _mod("_ops")
+    total, slack = prefix + tq, 37
+    rng = np.random.default_rng(tq + d)
+    r = lambda *s: torch.from_numpy(rng.standard_normal(s).astype(np.float32)).to(gpu)  # noqa: E731
+    q, K, V = r(tq, hq, d), r(total + slack, hkv, d), r(total + slack, hkv, d)
+    call = lambda k, v: P.prefill(q, k, v, pos0=prefix, window=window,  # noqa: E731
+                                  kv_tokens=total + slack)
+    clean = call(K, V)
+    Kb, Vb = K.clone(), V.clone()
+    Kb[total:], Vb[total:] = float("nan"), float("nan")
+    assert torch.equal(call(Kb, Vb), clean)
+    Kb[total - 1], Vb[total - 1, :, 1::2] = float("nan"), float("inf")
+    assert torch.equal(call(Kb, Vb)[:-1], clean[:-1])
+    Vb[total - 3, :, ::3] = float("-inf")
+    got = call(K, Vb)
+    assert torch.equal(got[:-3], clean[:-3])
+    assert bool(torch.isinf(got[-3, :, ::3]).all())
+
+
 def test_prefill_append_range_error_leaves_cache(gpu):
     import torch
     P = _mod("_ops")
