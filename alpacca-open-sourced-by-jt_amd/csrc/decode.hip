@@ -40,6 +40,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "alpx_common.h"
 #include "decode_internal.h"
@@ -385,7 +386,13 @@ __device__ __forceinline__ void write_out(const DecodeArgs& a, char* smem, f32x4
 // largest P is the exact 1 (bf16, rms of the result 1.2e-3 with one tile a
 // wave, 1.5e-3 with two to eight, 2e-6 in two parts): the kernels that give
 // a wave several tiles where shorter chunks gave it one take two parts.  It
-// costs 0.2-0.3 us of a 10 us step, also behind a branch.
+// costs 0.2-0.3 us of a 10 us step, also behind a branch.  The rest is 0 or
+// negative as often as not, and either times an infinity that the token sees
+// makes a NaN of it: a wave whose O is not finite walks its rows again, the
+// rests times the finite values only.  (A sum of their own for the rests,
+// joined where the first sum is finite, needs no second walk, but cost every
+// step of 4.5 to 20 us another 0.2 to 0.9; the test of O costs at most 0.1,
+// 0.2 at head_dim 256.)
 template <typename T, int D, bool PAGED, bool PRO, int NW, bool DIRECT, bool TWO>
 __device__ __forceinline__ void split_body(const DecodeArgs& a, const SplitPrologue* pp) {
   typedef typename Vec8<T>::type V8;
@@ -506,122 +513,156 @@ __device__ __forceinline__ void split_body(const DecodeArgs& a, const SplitProlo
   T* ldsk = (T*)smem + 2 * wave * kTileElems;
   T* ldsv = ldsk + kTileElems;
 
-  V8 kr[kIters];  // K rows, 16 bytes per lane, row-major
-  V8 vr[kIters];  // V rows, same layout
-  // Tile loads are raw buffer loads from the tile's first row: load `it`
-  // covers rows kRowsPerLoad * it + lane / kUnits, 16-byte unit lane %
-  // kUnits, so a lane's byte offset is its base plus it * (row step), one
-  // add per load.  The buffer ends at row `end`: rows past it read as zero
-  // (their scores are masked, their P is zero).
-  constexpr int kRowsPerLoad = 64 / kUnits;
-  const uint32_t koff = (uint32_t)(((lane / kUnits) * a.ks_pos + 8 * (lane % kUnits)) * (int64_t)sizeof(T));
-  const uint32_t voff = (uint32_t)(((lane / kUnits) * a.vs_pos + 8 * (lane % kUnits)) * (int64_t)sizeof(T));
-  const uint32_t kstep = (uint32_t)(kRowsPerLoad * a.ks_pos * (int64_t)sizeof(T));
-  const uint32_t vstep = (uint32_t)(kRowsPerLoad * a.vs_pos * (int64_t)sizeof(T));
-  auto load_tile = [&](int p) {
-    // Paged: a wave tile starts at a multiple of kTile and never crosses a
-    // page (page size a multiple of kTile), so its page is looked up once.
-    const T* kt = kbase + (int64_t)p * a.ks_pos;
-    const T* vt = vbase + (int64_t)p * a.vs_pos;
-    if constexpr (PAGED) {
-      kt = (const T*)a.k + row_offset(a, b, kvh, p, a.ks_pos, 0, a.ks_h, a.ks_page);
-      vt = (const T*)a.v + row_offset(a, b, kvh, p, a.vs_pos, 0, a.vs_h, a.vs_page);
-    }
-    const int rows = min(end - p, kTile);
-    const __amdgpu_buffer_rsrc_t kres = buffer_rsrc(kt, (uint32_t)(rows * a.ks_pos * (int64_t)sizeof(T)));
-    const __amdgpu_buffer_rsrc_t vres = buffer_rsrc(vt, (uint32_t)(rows * a.vs_pos * (int64_t)sizeof(T)));
+  // One walk over the wave's rows.  `lane` is a parameter, and opaque for the
+  // second walk, so that the two share no addresses: held for both, they
+  // pushed the first walk's into other registers.  At head_dim 256, where
+  // the loop has no register to spare, the scheduler then issued a tile's
+  // loads in another order than the loop stages them, which exposed them all
+  // (64 sequences of 1024 rows, 16/2 heads: 27.7 -> 35.5 us): the loads are
+  // kept in order there, two of each at a time (27.9; one 29.1).
+  auto walk = [&](auto again, const int lane) __attribute__((always_inline)) {
+    [[maybe_unused]] constexpr bool kAgain = decltype(again)::value;
+    const int hl = lane & 15, quad = lane >> 4;
+    V8 kr[kIters];  // K rows, 16 bytes per lane, row-major
+    V8 vr[kIters];  // V rows, same layout
+    // Tile loads are raw buffer loads from the tile's first row: load `it`
+    // covers rows kRowsPerLoad * it + lane / kUnits, 16-byte unit lane %
+    // kUnits, so a lane's byte offset is its base plus it * (row step), one
+    // add per load.  The buffer ends at row `end`: rows past it read as zero
+    // (their scores are masked, their P is zero).
+    constexpr int kRowsPerLoad = 64 / kUnits;
+    const uint32_t koff = (uint32_t)(((lane / kUnits) * a.ks_pos + 8 * (lane % kUnits)) * (int64_t)sizeof(T));
+    const uint32_t voff = (uint32_t)(((lane / kUnits) * a.vs_pos + 8 * (lane % kUnits)) * (int64_t)sizeof(T));
+    const uint32_t kstep = (uint32_t)(kRowsPerLoad * a.ks_pos * (int64_t)sizeof(T));
+    const uint32_t vstep = (uint32_t)(kRowsPerLoad * a.vs_pos * (int64_t)sizeof(T));
+    auto load_tile = [&](int p) {
+      // Paged: a wave tile starts at a multiple of kTile and never crosses a
+      // page (page size a multiple of kTile), so its page is looked up once.
+      const T* kt = kbase + (int64_t)p * a.ks_pos;
+      const T* vt = vbase + (int64_t)p * a.vs_pos;
+      if constexpr (PAGED) {
+        kt = (const T*)a.k + row_offset(a, b, kvh, p, a.ks_pos, 0, a.ks_h, a.ks_page);
+        vt = (const T*)a.v + row_offset(a, b, kvh, p, a.vs_pos, 0, a.vs_h, a.vs_page);
+      }
+      const int rows = min(end - p, kTile);
+      const __amdgpu_buffer_rsrc_t kres = buffer_rsrc(kt, (uint32_t)(rows * a.ks_pos * (int64_t)sizeof(T)));
+      const __amdgpu_buffer_rsrc_t vres = buffer_rsrc(vt, (uint32_t)(rows * a.vs_pos * (int64_t)sizeof(T)));
 #pragma unroll
-    for (int it = 0; it < kIters; ++it) {
-      kr[it] = __builtin_bit_cast(V8, __builtin_amdgcn_raw_buffer_load_b128(kres, koff + it * kstep, 0, 0));
-      vr[it] = __builtin_bit_cast(
-          V8, __builtin_amdgcn_raw_buffer_load_b128(vres, voff + it * vstep, 0, kAuxNontemporal));
-    }
-  };
+      for (int it = 0; it < kIters; ++it) {
+        kr[it] = __builtin_bit_cast(V8, __builtin_amdgcn_raw_buffer_load_b128(kres, koff + it * kstep, 0, 0));
+        vr[it] = __builtin_bit_cast(
+            V8, __builtin_amdgcn_raw_buffer_load_b128(vres, voff + it * vstep, 0, kAuxNontemporal));
+        if (TWO && D == 256 && it % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+      }
+    };
 
-  int p0 = start + kTile * wave;
-  if (p0 < end) load_tile(p0);
-  while (p0 < end) {
-    const int pn = p0 + kTile * NW;
-    // Stage K and V in LDS (row-major, padded rows), then prefetch the next tile.
+    int p0 = start + kTile * wave;
+    if (p0 < end) load_tile(p0);
+    while (p0 < end) {
+      const int pn = p0 + kTile * NW;
+      // Stage K and V in LDS (row-major, padded rows), then prefetch the next tile.
 #pragma unroll
-    for (int it = 0; it < kIters; ++it) {
-      const int u = it * 64 + lane;
-      const int r = u / kUnits;
-      const int c = u - r * kUnits;
-      *(V8*)(ldsk + r * kStride + 8 * c) = kr[it];
-      *(V8*)(ldsv + r * kStride + 8 * c) = vr[it];
-    }
-    if constexpr (PRO) {
-      const int64_t r = (pp->positions ? (int64_t)pp->positions[b] : pp->position) - p0;
-      if (owns_new && r >= 0 && r < kTile) {
-        for (int i = lane; i < D; i += 64) {
-          ldsk[r * kStride + i] = new_kv[i];
-          ldsv[r * kStride + i] = new_kv[D + i];
+      for (int it = 0; it < kIters; ++it) {
+        const int u = it * 64 + lane;
+        const int r = u / kUnits;
+        const int c = u - r * kUnits;
+        *(V8*)(ldsk + r * kStride + 8 * c) = kr[it];
+        *(V8*)(ldsv + r * kStride + 8 * c) = vr[it];
+      }
+      if constexpr (PRO) {
+        const int64_t r = (pp->positions ? (int64_t)pp->positions[b] : pp->position) - p0;
+        if (owns_new && r >= 0 && r < kTile) {
+          for (int i = lane; i < D; i += 64) {
+            ldsk[r * kStride + i] = new_kv[i];
+            ldsv[r * kStride + i] = new_kv[D + i];
+          }
         }
       }
-    }
-    if (pn < end) load_tile(pn);
-    wave_sync_lds();
-    // Scores for 32 rows x 16 heads: lane holds S[pos = p0 + 16 blk + 4 quad + i][hl].
-    f32x4 s[2];
+      if (pn < end) load_tile(pn);
+      wave_sync_lds();
+      // Scores for 32 rows x 16 heads: lane holds S[pos = p0 + 16 blk + 4 quad + i][hl].
+      f32x4 s[2];
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
-      s[blk] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      for (int blk = 0; blk < 2; ++blk) {
+        s[blk] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < D / 32; ++ks) {
-        const V8 ka = *(const V8*)(ldsk + (16 * blk + hl) * kStride + 32 * ks + 8 * quad);
-        s[blk] = mfma16x16x32(ka, qv[ks], s[blk]);
+        for (int ks = 0; ks < D / 32; ++ks) {
+          const V8 ka = *(const V8*)(ldsk + (16 * blk + hl) * kStride + 32 * ks + 8 * quad);
+          s[blk] = mfma16x16x32(ka, qv[ks], s[blk]);
+        }
       }
-    }
-    // Online softmax (base 2).  Slot j of this lane is row 16 (j/4) + 4 quad + j%4.
-    float sv[8];
-    float mx = -INFINITY;
+      // Online softmax (base 2).  Slot j of this lane is row 16 (j/4) + 4 quad + j%4.
+      float sv[8];
+      float mx = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int pos = p0 + 16 * (j >> 2) + 4 * quad + (j & 3);
-      const float x = pos < end ? s[j >> 2][j & 3] * a.scale_log2 : -INFINITY;
-      sv[j] = x;
-      mx = fmaxf(mx, x);
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    // Lazy reference max: m moves only when the tile's max exceeds it by
-    // more than kDecodeRescale (so P <= 2^kDecodeRescale), and O is rescaled
-    // only on a step where some head of the wave moved.  Every tile holds at
-    // least one live row, so the first tile always moves m off -inf.
-    const bool grow = mx > m + kDecodeRescale;
-    const float mn = grow ? mx : m;
-    const float alpha = grow ? fast_exp2(m - mn) : 1.f;
-    V8 pv;
-    [[maybe_unused]] V8 pr;
-    float ps = 0.f;
+      for (int j = 0; j < 8; ++j) {
+        const int pos = p0 + 16 * (j >> 2) + 4 * quad + (j & 3);
+        const float x = pos < end ? s[j >> 2][j & 3] * a.scale_log2 : -INFINITY;
+        sv[j] = x;
+        mx = fmaxf(mx, x);
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      // Lazy reference max: m moves only when the tile's max exceeds it by
+      // more than kDecodeRescale (so P <= 2^kDecodeRescale), and O is rescaled
+      // only on a step where some head of the wave moved.  Every tile holds at
+      // least one live row, so the first tile always moves m off -inf.
+      const bool grow = mx > m + kDecodeRescale;
+      const float mn = grow ? mx : m;
+      const float alpha = grow ? fast_exp2(m - mn) : 1.f;
+      V8 pv;
+      [[maybe_unused]] V8 pr;
+      float ps = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float p = fast_exp2(sv[j] - mn);
-      ps += p;
-      pv[j] = from_f32<T>(p);
-      if constexpr (TWO) pr[j] = from_f32<T>(p - to_f32(pv[j]));
-    }
-    l = l * alpha + ps;
-    m = mn;
-    if (__builtin_expect(__ballot(grow) != 0, 0)) {
+      for (int j = 0; j < 8; ++j) {
+        const float p = fast_exp2(sv[j] - mn);
+        ps += p;
+        pv[j] = from_f32<T>(p);
+        if constexpr (TWO) pr[j] = from_f32<T>(p - to_f32(pv[j]));
+      }
+      l = l * alpha + ps;
+      m = mn;
+      if (__builtin_expect(__ballot(grow) != 0, 0)) {
 #pragma unroll
-      for (int mb = 0; mb < D / 16; ++mb) o[mb] *= alpha;
-    }
-    // O^T += V^T P^T.  A operand: lane holds V[row(quad, j)][16 mb + hl], j = 0..7,
-    // gathered with two transposing reads of 4 rows (16 h + 4 quad + 0..3) each.
-    const int tr_row = 4 * quad + (hl >> 2);
-    const int tr_col = 4 * (hl & 3);
+        for (int mb = 0; mb < D / 16; ++mb) o[mb] *= alpha;
+      }
+      // O^T += V^T P^T.  A operand: lane holds V[row(quad, j)][16 mb + hl], j = 0..7,
+      // gathered with two transposing reads of 4 rows (16 h + 4 quad + 0..3) each.
+      const int tr_row = 4 * quad + (hl >> 2);
+      const int tr_col = 4 * (hl & 3);
 #pragma unroll
-    for (int mb = 0; mb < D / 16; ++mb) {
-      const V4 lo = lds_read_tr4(ldsv + tr_row * kStride + 16 * mb + tr_col);
-      const V4 hi = lds_read_tr4(ldsv + (16 + tr_row) * kStride + 16 * mb + tr_col);
-      const V8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-      if constexpr (TWO) o[mb] = mfma16x16x32(va, pr, o[mb]);
-      o[mb] = mfma16x16x32(va, pv, o[mb]);
+      for (int mb = 0; mb < D / 16; ++mb) {
+        const V4 lo = lds_read_tr4(ldsv + tr_row * kStride + 16 * mb + tr_col);
+        const V4 hi = lds_read_tr4(ldsv + (16 + tr_row) * kStride + 16 * mb + tr_col);
+        const V8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        if constexpr (TWO) {
+          V8 vf = va;
+          if constexpr (kAgain) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) vf[j] = fabsf(to_f32(va[j])) < INFINITY ? va[j] : (T)0;
+          }
+          o[mb] = mfma16x16x32(vf, pr, o[mb]);
+        }
+        o[mb] = mfma16x16x32(va, pv, o[mb]);
+      }
+      wave_sync_lds();
+      p0 = pn;
     }
-    wave_sync_lds();
-    p0 = pn;
+  };
+  walk(std::false_type(), lane);
+  if constexpr (TWO) {
+    f32x4 z = {0.f, 0.f, 0.f, 0.f};  // stays 0 while O is finite
+#pragma unroll
+    for (int mb = 0; mb < D / 16; ++mb) z += 0.f * o[mb];
+    if (__builtin_expect(__ballot(!(z[0] + z[1] + z[2] + z[3] == 0.f)) != 0, 0)) {
+#pragma unroll
+      for (int mb = 0; mb < D / 16; ++mb) o[mb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      m = -INFINITY;
+      l = 0.f;
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      walk(std::true_type(), ln);
+    }
   }
 
   if constexpr (DIRECT)

@@ -358,6 +358,63 @@ def test_decode_balanced_rounds(gpu, ops, hq, hkv, d, dtype, lens):
         assert err <= TOL[dtype], (b, err)
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("hq,hkv,d,lens,kind", [
+    (8, 2, 64, [512] * 2, "plain"), (8, 2, 64, [513] * 2, "plain"),       # one launch, two
+    (32, 8, 128, [384] * 3, "paged"), (32, 8, 128, [385] * 3, "paged"),
+    (34, 2, 256, [128] * 2, "plain"), (16, 2, 256, [129] * 2, "plain"),
+    (8, 2, 128, [120] * 2, "step"), (8, 2, 64, [100, 31], "ragged"),
+    (32, 8, 128, [3000, 77, 2200, 3], "ragged"),        # one round of blocks
+    (32, 8, 128, [5900, 6000, 5800, 6300], "ragged"),   # two and a half
+    (32, 8, 128, [3000, 77, 2200, 3], "paged"), (16, 2, 256, [14000, 15500, 90, 8000], "ragged")])
+def test_decode_seen_infinity_stays_one(gpu, ops, hq, hkv, d, lens, kind, dtype):
+    """An infinity in a value row that a token sees comes out as itself, as
+    the weighted sum has it, where P enters its product in one part and where
+    it does in two (one launch, one round): on both sides of their limits.
+    Every other channel and sequence keeps its bits."""
+    import torch
+    B, C = len(lens), max(lens)
+    gen = torch.Generator(device=gpu).manual_seed(C + d)
+    r = lambda *s: torch.randn(*s, generator=gen, device=gpu).to(_tdtype(torch, dtype))  # noqa: E731
+    q, K, V = r(B, hq, d), r(C, B, hkv, d), r(C, B, hkv, d)
+    seq = torch.tensor(lens, dtype=torch.int32, device=gpu)
+    page = 32
+    per = -(-C // page)
+    table = torch.randperm(B * per, generator=gen, device=gpu).to(torch.int32).reshape(B, per)
+    qg, kn, vn = r(B, hq * 2 * d), r(B, hkv * d), r(B, hkv * d)
+    w = torch.ones(d, device=gpu)
+
+    def call(V):
+        if kind == "step":
+            out, _ = ops.attention_layer_step_(qg, kn, vn, w, w, K.clone(), V.clone(),
+                                               position=C - 1, sections=(11, 11, 10, 0),
+                                               frequency_base=1e7, epsilon=1e-6)
+            return out.float().reshape(B, hq, d)
+        if kind == "paged":
+            pools = []
+            for x in (K, V):
+                pool = torch.zeros(B * per * page, hkv, d, dtype=x.dtype, device=gpu)
+                j = torch.arange(C, device=gpu)
+                for b in range(B):
+                    pool[table[b].long()[j // page] * page + j % page] = x[:, b]
+                pools.append(pool.reshape(B * per, page, hkv, d))
+            return ops.paged_online_attention(q, *pools, table, length=C, out_dtype=torch.float32,
+                                              seq_lens=seq)
+        return ops.online_attention(q, K, V, length=C, out_dtype=torch.float32,
+                                    seq_lens=seq if kind == "ragged" else None)
+
+    clean = call(V)
+    Vb = V.clone()
+    n = lens[0]
+    Vb[n // 2, 0, :, ::3] = float("inf")
+    Vb[n // 3, 0, :, 1::3] = float("-inf")
+    got = call(Vb)
+    assert torch.isfinite(clean).all()
+    assert bool((got[0, :, ::3] == float("inf")).all())
+    assert bool((got[0, :, 1::3] == float("-inf")).all())
+    assert torch.equal(got[0, :, 2::3], clean[0, :, 2::3]) and torch.equal(got[1:], clean[1:])
+
+
 def test_decode_repeatable_across_plans(gpu, ops):
     import torch
     rng = np.random.default_rng(11)
