@@ -143,16 +143,19 @@ def decode_paged(q, key_pages, value_pages, block_table, *, length, seq_lens=Non
     return out
 
 
+def _split_bytes(L, *sizes):
+    """``alpx_prefill_split_bytes(*sizes)``, which is 0 up to 480 cache rows
+    (8 key tiles of 64, 15 of 32): the shortest calls, bound by their host
+    time, don't ask."""
+    return L.alpx_prefill_split_bytes(*sizes) if sizes[1] > 480 else 0
+
+
 def _split_workspace(L, device, *sizes):
     """Workspace of its own for an MFMA prefill that cuts its key ranges over
     several blocks (None where the chunk runs unsplit): from torch's
     stream-ordered allocator, so that calls on different streams share
-    nothing.  ``sizes``: the arguments of alpx_prefill_split_bytes, which is
-    0 up to 480 cache rows (7 key tiles of 64, 15 of 32): the shortest
-    calls, bound by their host time, don't ask."""
-    if sizes[1] <= 480:
-        return None
-    nbytes = L.alpx_prefill_split_bytes(*sizes)
+    nothing.  ``sizes``: the arguments of alpx_prefill_split_bytes."""
+    nbytes = _split_bytes(L, *sizes)
     return _torch().empty(nbytes, dtype=_torch().uint8, device=device) if nbytes else None
 
 
@@ -792,18 +795,22 @@ def attention_layer_prefill(query_gate, key, value, q_norm, k_norm, key_cache, v
             _lib.stream_handle(torch, dev))
 
     # Every refusal below comes before the library's first launch, so a
-    # refused form has written nothing and the next form may run.
-    split = L.alpx_prefill_split_bytes(tokens, int(position) + tokens, q_heads, kv_heads, dim,
-                                       int(position), 0, 0) if fast else 0
+    # refused form has written nothing and the next form may run.  The
+    # rotation table and a split chunk's partials have a buffer of the call's
+    # own, as in prefill_append: calls on different streams share nothing.
+    def own(nbytes):
+        return torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes > 0 else None
+
+    split = _split_bytes(L, tokens, int(position) + tokens, q_heads, kv_heads, dim,
+                         int(position), 0, 0) if fast else 0
     if fused_query:
         table = (tokens * pairs * 8 + 255) // 256 * 256
-        rc = call(None, _lib.workspace(torch, dev, max(table + split, 1)))
+        rc = call(None, own(max(table + split, 1)))
         if not (auto and rc == _lib.EUNSUPPORTED):  # e.g. a cache of 2 GiB or more
             _lib.check(rc)
             return out
     query = torch.empty((tokens, q_heads, dim), dtype=key_cache.dtype, device=dev)
-    # its own, as in prefill_append: this form shares no workspace between streams
-    rc = call(query, torch.empty(split, dtype=torch.uint8, device=dev) if split else None)
+    rc = call(query, own(split))
     if rc == _lib.EINVAL:  # the split-K prefill (fp32, unaligned, >= 2 GiB) needs a workspace
         nbytes = L.alpx_prefill_workspace_bytes(tokens, q_heads, kv_heads, dim,
                                                 int(position) + tokens)

@@ -170,8 +170,10 @@ def test_attention_layer_prefill_equals_prologue_then_gated_prefill(gpu, hq, hkv
         assert torch.equal(out_a, out_b), fused
 
 
-def test_attention_layer_prefill_query_buffer_form_shares_no_workspace(gpu, monkeypatch):
-    """The query-buffer form of a chunk whose key ranges are split takes its
+@pytest.mark.parametrize("form", [False, True, None])
+def test_attention_layer_prefill_shares_no_workspace(gpu, monkeypatch, form):
+    """Each form of a chunk whose key ranges are split (the query buffer, the
+    fused query, the choice between them) takes the rotation table and its
     partials from a buffer of its own, so that calls on two streams share
     nothing."""
     import torch
@@ -185,13 +187,13 @@ def test_attention_layer_prefill_query_buffer_form_shares_no_workspace(gpu, monk
     args = (b(tokens, hq, 2 * d), b(tokens, hkv, d), b(tokens, hkv, d), r(d), r(d), kc, vc)
     kw = dict(batch_index=0, position=prefix, sections=(11, 11, 10, 0), frequency_base=1e6,
               eps=1e-6)
-    fused = P.attention_layer_prefill(*args, fused_query=True, **kw)
+    ref = P.attention_layer_prefill(*args, fused_query=form is False, **kw)
 
     def shared(*_):
         raise AssertionError("the shared workspace was taken")
 
     monkeypatch.setattr(Lib, "workspace", shared)
-    assert torch.equal(P.attention_layer_prefill(*args, fused_query=False, **kw), fused)
+    assert torch.equal(P.attention_layer_prefill(*args, fused_query=form, **kw), ref)
 
 
 def test_attention_layer_prefill_cache_of_2gib_or_more(gpu, ops):
