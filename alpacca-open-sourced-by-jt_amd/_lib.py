@@ -69,6 +69,8 @@ SIGNATURES = {
                                            _c_size, _c_int, _c_int, _c_int, _c_int, _c_int,
                                            _c_int, _c_i64, _c_i64, _c_i64, _c_int, _c_i64,
                                            _c_float, _c_int, _c_int, _c_ptr]),
+    "alpx_prefill_f32_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
+                                                   _c_i64, _c_int, _c_i64, _c_ptr]),
     "alpx_prefill_split_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_i64, _c_int,
                                            _c_i64]),
     "alpx_prefill_append": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,

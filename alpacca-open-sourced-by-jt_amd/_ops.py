@@ -8,6 +8,7 @@ in libalpx.so.  Nothing here computes on the CPU.
 
 from __future__ import annotations
 
+import functools
 import math
 
 from . import _lib
@@ -159,6 +160,14 @@ def _split_workspace(L, device, *sizes):
     return _torch().empty(nbytes, dtype=_torch().uint8, device=device) if nbytes else None
 
 
+@functools.lru_cache(maxsize=1024)
+def _f32_prefill_bytes(*sizes):
+    """``alpx_prefill_f32_workspace_bytes``, a pure function of the sizes.
+    float32 calls bring what their plan wants and no more, however large the
+    shared buffer has grown: the plan follows the bytes."""
+    return _lib.lib().alpx_prefill_f32_workspace_bytes(*sizes, None)
+
+
 def prefill_append(q, key, value, key_cache, value_cache, *, position, scale=None, window=0,
                    out_dtype=None, gate=None):
     """Writes the chunk's rows ``key/value [T, Hkv, D]`` to rows ``position ..``
@@ -174,31 +183,34 @@ def prefill_append(q, key, value, key_cache, value_cache, *, position, scale=Non
     out_dtype = q.dtype if out_dtype is None else out_dtype
     out = torch.empty((q_tokens, q_heads, value_dim), dtype=out_dtype, device=q.device)
     L = _lib.lib()
-    nbytes = L.alpx_prefill_workspace_bytes(q_tokens, q_heads, kv_heads, value_dim,
-                                            int(position) + q_tokens)
+    f32 = q.dtype == torch.float32
+    total = int(position) + q_tokens
+    nbytes = (_f32_prefill_bytes(q_tokens, total, q_heads, kv_heads, key_dim, value_dim,
+                                 int(position), int(window), 0)
+              if f32 else L.alpx_prefill_workspace_bytes(q_tokens, q_heads, kv_heads, value_dim,
+                                                         total))
     if nbytes == 0:
         raise ValueError("invalid prefill sizes")
-    fast = (q.dtype != torch.float32 and key_dim == value_dim and key_dim in (64, 128, 256))
-    ws = (_split_workspace(L, q.device, q_tokens, int(position) + q_tokens, q_heads, kv_heads,
-                           key_dim, int(position), int(window), 0)
+    fast = (not f32 and key_dim == value_dim and key_dim in (64, 128, 256))
+    ws = (_split_workspace(L, q.device, q_tokens, total, q_heads, kv_heads, key_dim,
+                           int(position), int(window), 0)
           if fast else _lib.workspace(torch, q.device, nbytes))
 
-    def call(workspace):
+    def call(workspace, size):
         return L.alpx_prefill_append(
             q.data_ptr(), key.data_ptr(), value.data_ptr(), key_cache.data_ptr(),
             value_cache.data_ptr(), None if gate is None else gate.data_ptr(), out.data_ptr(),
-            None if workspace is None else workspace.data_ptr(),
-            0 if workspace is None else workspace.numel(), q_tokens, capacity, q_heads, kv_heads,
-            key_dim, value_dim, int(position), int(window), float(scale),
+            None if workspace is None else workspace.data_ptr(), size, q_tokens, capacity, q_heads,
+            kv_heads, key_dim, value_dim, int(position), int(window), float(scale),
             _lib.dtype_code(torch, q.dtype), _lib.dtype_code(torch, out.dtype),
             _lib.stream_handle(torch, q.device))
 
-    rc = call(ws)
+    rc = call(ws, nbytes if not fast else (0 if ws is None else ws.numel()))
     # unaligned rows or a cache of 2 GiB or more leave the MFMA kernels; the
     # split-K path refuses a null or small workspace before its append
     if rc == _lib.EINVAL and fast:
         ws = _lib.workspace(torch, q.device, nbytes)
-        rc = call(ws)
+        rc = call(ws, nbytes)
     _lib.check(rc)
     return out
 
@@ -413,31 +425,34 @@ def prefill(q, key, value, *, pos0, scale=None, window=0, kv_start=0, kv_tokens=
     if out is None:
         out = torch.empty((q_tokens, q_heads, value_dim), dtype=out_dtype, device=q.device)
     L = _lib.lib()
-    nbytes = L.alpx_prefill_workspace_bytes(q_tokens, q_heads, kv_heads, value_dim, kv_tokens)
+    f32 = q.dtype == torch.float32
+    nbytes = (_f32_prefill_bytes(q_tokens, int(kv_tokens), q_heads, kv_heads, key_dim, value_dim,
+                                 int(pos0), int(window), int(kv_start))
+              if f32 else L.alpx_prefill_workspace_bytes(q_tokens, q_heads, kv_heads, value_dim,
+                                                         int(kv_tokens)))
     if nbytes == 0:
         raise ValueError("invalid prefill sizes")
-    # the split-K fallback (fp32, odd shapes) needs the workspace
-    fast = (q.dtype != torch.float32 and key_dim == value_dim and key_dim in (64, 128, 256))
+    # float32 and the split-K fallback (odd shapes) need the workspace
+    fast = (not f32 and key_dim == value_dim and key_dim in (64, 128, 256))
     ws = (_split_workspace(L, q.device, q_tokens, int(kv_tokens), q_heads, kv_heads, key_dim,
                            int(pos0), int(window), int(kv_start))
           if fast else _lib.workspace(torch, q.device, nbytes))
 
-    def call(workspace):
-        args = (None if workspace is None else workspace.data_ptr(),
-                0 if workspace is None else workspace.numel(), q_tokens, int(kv_tokens), q_heads,
-                kv_heads, key_dim, value_dim, int(k_pos_stride), int(v_pos_stride), int(pos0),
-                int(window), int(kv_start), float(scale), _lib.dtype_code(torch, q.dtype),
-                _lib.dtype_code(torch, out.dtype), _lib.stream_handle(torch, q.device))
+    def call(workspace, size):
+        args = (None if workspace is None else workspace.data_ptr(), size, q_tokens,
+                int(kv_tokens), q_heads, kv_heads, key_dim, value_dim, int(k_pos_stride),
+                int(v_pos_stride), int(pos0), int(window), int(kv_start), float(scale),
+                _lib.dtype_code(torch, q.dtype), _lib.dtype_code(torch, out.dtype), _lib.stream_handle(torch, q.device))
         if gate is None:
             return L.alpx_prefill_causal(q.data_ptr(), key.data_ptr(), value.data_ptr(),
                                          out.data_ptr(), *args)
         return L.alpx_prefill_causal_gated(q.data_ptr(), key.data_ptr(), value.data_ptr(),
                                            gate.data_ptr(), out.data_ptr(), *args)
 
-    rc = call(ws)
+    rc = call(ws, nbytes if not fast else (0 if ws is None else ws.numel()))
     if rc == _lib.EINVAL and fast:  # unaligned rows fell back: retry with its workspace
         ws = _lib.workspace(torch, q.device, nbytes)
-        rc = call(ws)
+        rc = call(ws, nbytes)
     _lib.check(rc)
     return out
 
@@ -783,12 +798,13 @@ def attention_layer_prefill(query_gate, key, value, q_norm, k_norm, key_cache, v
         fused_query = (fast and pairs % 32 == 0 and 2 * pairs <= dim
                        and _lib.get_override(_lib.OVERRIDE_PREFILL_GENERIC) == 0)
 
-    def call(query, ws):
+    def call(query, ws, size=None):
         return L.alpx_attention_layer_prefill(
             query_gate.data_ptr(), key.data_ptr(), value.data_ptr(), q_norm.data_ptr(),
             k_norm.data_ptr(), None if query is None else query.data_ptr(),
             key_cache.data_ptr(), value_cache.data_ptr(), out.data_ptr(),
-            None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
+            None if ws is None else ws.data_ptr(),
+            size if size is not None else (0 if ws is None else ws.numel()),
             _lib.dtype_code(torch, key_cache.dtype), _lib.dtype_code(torch, out.dtype), capacity,
             cache_batch, int(batch_index), tokens, q_heads, kv_heads, dim, int(position),
             _sections(sections), float(frequency_base), float(eps), float(scale),
@@ -812,11 +828,13 @@ def attention_layer_prefill(query_gate, key, value, q_norm, k_norm, key_cache, v
     query = torch.empty((tokens, q_heads, dim), dtype=key_cache.dtype, device=dev)
     rc = call(query, own(split))
     if rc == _lib.EINVAL:  # the split-K prefill (fp32, unaligned, >= 2 GiB) needs a workspace
-        nbytes = L.alpx_prefill_workspace_bytes(tokens, q_heads, kv_heads, dim,
-                                                int(position) + tokens)
+        total = int(position) + tokens
+        nbytes = (_f32_prefill_bytes(tokens, total, q_heads, kv_heads, dim, dim, int(position), 0, 0)
+                  if key_cache.dtype == torch.float32
+                  else L.alpx_prefill_workspace_bytes(tokens, q_heads, kv_heads, dim, total))
         if nbytes == 0:
             raise ValueError("invalid prefill sizes")
-        rc = call(query, _lib.workspace(torch, dev, nbytes))
+        rc = call(query, _lib.workspace(torch, dev, nbytes), nbytes)
     _lib.check(rc)
     return out
 

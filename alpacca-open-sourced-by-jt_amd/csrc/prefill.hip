@@ -182,8 +182,11 @@ SplitPlan plan_split_prefill(int q_tokens, int kv_tokens, int q_heads, int kv_he
 // 25 / 18 (32 pieces), 1 on 4096 12 / 12; head_dim 128, 1000 on 4096
 // 3325 / 599, 4 on 1024 22 / 16, 1 on 4096 16 / 25; head_dim 256, 700 on
 // 4096 1518 / 485 (4 pieces), 9 on 4096 33 / 42.
+// Among the splits whose partials fit `limit` bytes: 300 tokens on 100 rows
+// of 8/8 heads of 128 want 7 pieces, 9.3 MB, where the decode machinery (91
+// us in place of 11) needs 8.7.
 SplitPlan plan_split_f32(int q_tokens, int kv_tokens, int kv_heads, int group, int head_dim,
-                         int rel0, int window) {
+                         int rel0, int window, size_t limit) {
   SplitPlan p = {0, 0, 0, 0};
   const int rows = head_dim == 256 ? 16 : 32;
   const double pair_us = head_dim == 64 ? 2.2 : (head_dim == 128 ? 4.1 : 4.4);
@@ -214,19 +217,15 @@ SplitPlan plan_split_f32(int q_tokens, int kv_tokens, int kv_heads, int group, i
     const int n = (most + c - 1) / c;
     const double blocks = std::min<double>(items * (double)n, items * (avg / c + 0.5));
     const double us = combine_us + blocks * 64 * head_dim * 8 / 4e6 + walk_us(c, blocks);
-    if (us < best) {
+    const size_t slots = (size_t)items * n;
+    const size_t o_bytes = slots * 64 * head_dim * sizeof(float);
+    const size_t bytes = o_bytes + slots * 64 * sizeof(float2);
+    if (us < best && bytes <= limit) {
       best = us;
-      p.splits = n;
-      p.split_tiles = c;
+      p = {n, c, o_bytes, bytes};
     }
   }
-  if (decode_us < 1.1 * best) {
-    p.splits = -1;
-  } else if (p.splits > 0) {
-    const size_t slots = (size_t)items * p.splits;
-    p.o_bytes = slots * 64 * head_dim * sizeof(float);
-    p.bytes = p.o_bytes + slots * 64 * sizeof(float2);
-  }
+  if (decode_us < 1.1 * best) p = {-1, 0, 0, 0};
   return p;
 }
 
@@ -471,8 +470,9 @@ int prefill_impl(const void* q, const void* key, const void* value, const void* 
       flash_operands(dtype, key_dim, value_dim, align, kv_tokens, k_pos_stride, v_pos_stride,
                      q_pos0 - kv_start)) {
     const SplitPlan sp = plan_split_f32(q_tokens, kv_tokens, kv_heads, group, key_dim,
-                                        (int)(q_pos0 - kv_start), window);
-    if (sp.splits >= 0 && ((uintptr_t)workspace & 15) == 0 && sp.bytes <= workspace_bytes) {
+                                        (int)(q_pos0 - kv_start), window,
+                                        ((uintptr_t)workspace & 15) == 0 ? workspace_bytes : 0);
+    if (sp.splits >= 0) {
       const bool split = sp.splits > 0;
       a.col_tiles = (int)(((int64_t)q_tokens * group + 63) / 64);
       a.splits = sp.splits;
@@ -536,6 +536,23 @@ extern "C" size_t alpx_prefill_split_bytes(int q_tokens, int kv_tokens, int q_he
       window < 0 || rel0 >= ((int64_t)1 << 30) || rel0 <= -((int64_t)1 << 30))
     return 0;
   return plan_split_prefill(q_tokens, kv_tokens, q_heads, kv_heads, head_dim, rel0, window).bytes;
+}
+
+extern "C" size_t alpx_prefill_f32_workspace_bytes(int q_tokens, int kv_tokens, int q_heads,
+                                                   int kv_heads, int key_dim, int value_dim,
+                                                   int64_t q_pos0, int window, int64_t kv_start,
+                                                   int* pieces) {
+  const size_t need =
+      alpx_prefill_workspace_bytes(q_tokens, q_heads, kv_heads, value_dim, kv_tokens);
+  const int64_t rel0 = q_pos0 - kv_start;
+  SplitPlan p = {-1, 0, 0, 0};
+  if (need > 0 && key_dim == value_dim && (key_dim == 64 || key_dim == 128 || key_dim == 256) &&
+      window >= 0 && rel0 < ((int64_t)1 << 30) && rel0 > -((int64_t)1 << 30) &&
+      (int64_t)q_tokens * (q_heads / kv_heads) < ((int64_t)1 << 30))
+    p = plan_split_f32(q_tokens, kv_tokens, kv_heads, q_heads / kv_heads, key_dim, (int)rel0,
+                       window, SIZE_MAX);
+  if (pieces != nullptr) *pieces = p.splits;
+  return std::max(need, p.bytes);
 }
 
 extern "C" int alpx_prefill_causal(const void* q, const void* key, const void* value, void* out,

@@ -249,11 +249,25 @@ int alpx_decode_gqa_noalloc(const void* q, const void* key_cache, const void* va
                             float scale, int dtype, int out_dtype, void* stream);
 
 /*
- * Workspace bytes alpx_prefill_causal may need (only its fallback path, for
- * fp32 or unsupported shapes, uses it).
+ * Workspace bytes alpx_prefill_causal may need (only float32 and its
+ * fallback path, for unsupported shapes, use it).
  */
 size_t alpx_prefill_workspace_bytes(int q_tokens, int q_heads, int kv_heads, int value_dim,
                                     int kv_tokens);
+
+/*
+ * Workspace bytes with which a float32 chunk runs its fastest plan: at least
+ * alpx_prefill_workspace_bytes, and more where it cuts its key ranges into
+ * more pieces than fit those.  A call that brings less takes the fastest
+ * plan that fits (the same result within rounding), so calls that have to
+ * agree bit for bit bring this much, whatever else their buffer holds.
+ * pieces (host memory, may be null): pieces of key ranges, merged by a second
+ * launch; 0 whole key ranges; -1 the split-K machinery (a few tokens on a long
+ * prefix, head dims other than 64, 128 and 256).  0 for invalid sizes.
+ */
+size_t alpx_prefill_f32_workspace_bytes(int q_tokens, int kv_tokens, int q_heads, int kv_heads,
+                                        int key_dim, int value_dim, int64_t q_pos0, int window,
+                                        int64_t kv_start, int* pieces);
 
 /*
  * Workspace bytes with which the MFMA prefill (alpx_prefill_causal,
@@ -286,8 +300,11 @@ size_t alpx_prefill_split_bytes(int q_tokens, int kv_tokens, int q_heads, int kv
  * seam's convention, cuda.py:572-577).  Scale is usually 1/sqrt(key_dim).
  * fp16/bf16 with key_dim == value_dim in {64, 128, 256} and 16-byte aligned
  * rows run the MFMA flash kernel (which needs no workspace and takes
- * alpx_prefill_split_bytes of it where given); anything else runs the
- * split-K machinery and needs alpx_prefill_workspace_bytes of workspace.
+ * alpx_prefill_split_bytes of it where given); anything else needs
+ * alpx_prefill_workspace_bytes of workspace.  Of that, float32 with the same
+ * head dims and alignment runs the float32 MFMA kernel (given
+ * alpx_prefill_f32_workspace_bytes, in as many pieces as are fastest), and
+ * the rest the split-K machinery.
  */
 int alpx_prefill_causal(const void* q, const void* key, const void* value, void* out,
                         void* workspace, size_t workspace_bytes, int q_tokens, int kv_tokens,

@@ -98,6 +98,17 @@ def test_decode_workspace_sizes(pkg):
     # grows with the number of partial slots, never below the 1-slot size
     one = 3 * 256
     assert lib.alpx_decode_workspace_bytes(1, 1, 1, 64, 1) >= one
+    # float32 chunks: at least the common size, whatever the plan
+    pieces = ctypes.c_int(7)
+    for t, kv, hq, hkv, dk, dv in ((300, 400, 8, 8, 128, 128), (16, 1516, 8, 8, 64, 64),
+                                   (9, 40, 8, 2, 64, 32), (1, 4096, 4, 1, 128, 128)):
+        need = lib.alpx_prefill_workspace_bytes(t, hq, hkv, dv, kv)
+        args = (t, kv, hq, hkv, dk, dv, kv - t, 0, 0)
+        size = lib.alpx_prefill_f32_workspace_bytes(*args, ctypes.byref(pieces))
+        assert size >= need > 0 and (size == need or pieces.value > 1)
+        assert lib.alpx_prefill_f32_workspace_bytes(*args, None) == size
+    assert pieces.value == -1
+    assert lib.alpx_prefill_f32_workspace_bytes(0, 1, 1, 1, 64, 64, 0, 0, 0, None) == 0
 
 
 def test_workspace_growth_is_geometric_and_caches_are_bounded(pkg):

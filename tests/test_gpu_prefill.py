@@ -280,6 +280,63 @@ def test_prefill_f32_unseen_rows_never_reach_a_row(gpu, tq, prefix, hq, hkv, d, 
     assert bool(torch.isinf(got[-3, :, ::3]).all())
 
 
+@pytest.mark.parametrize("tq,prefix,hq,hkv,d,least_runs", [
+    (300, 100, 8, 8, 128, "f32"), (634, 0, 8, 8, 64, "f32"), (16, 1500, 8, 8, 64, "decode"),
+    (90, 300, 8, 8, 256, "f32")])
+def test_prefill_f32_plan_follows_the_call_not_the_workspace(gpu, monkeypatch, tq, prefix, hq,
+                                                             hkv, d, least_runs):
+    """Float32 chunks whose fastest plan needs more partials than the decode
+    machinery: the facade's call gives the same bits in a fresh process and
+    after a larger call has grown the shared workspace, and those of the
+    library call that brings the queried bytes.  One that brings only
+    alpx_prefill_workspace_bytes runs the float32 kernel in fewer pieces (no
+    combine launch of the decode machinery), except the few tokens that then
+    are the decode machinery's."""
+    import ctypes
+
+    import torch
+    P, Lib = _mod("_ops"), _mod("_lib")
+    lib = Lib.lib()
+    total, scale = prefix + tq, 1.0 / np.sqrt(d)
+    pieces = ctypes.c_int()
+    want = lib.alpx_prefill_f32_workspace_bytes(tq, total, hq, hkv, d, d, prefix, 0, 0,
+                                                ctypes.byref(pieces))
+    least = lib.alpx_prefill_workspace_bytes(tq, hq, hkv, d, total)
+    assert pieces.value > 1 and want > least
+    gen = torch.Generator(device=gpu).manual_seed(tq)
+    r = lambda *s: torch.randn(*s, generator=gen, device=gpu)  # noqa: E731
+    q, K, V = r(tq, hq, d), r(total, hkv, d), r(total, hkv, d)
+    for name in ("_workspaces", "_workspace_bytes", "_retired"):
+        monkeypatch.setattr(Lib, name, {})
+    fresh = P.prefill(q, K, V, pos0=prefix)
+    Lib.workspace(torch, gpu, 4 * want)
+    assert torch.equal(P.prefill(q, K, V, pos0=prefix), fresh)
+
+    def call(nbytes):
+        ws, out = torch.empty(nbytes, dtype=torch.uint8, device=gpu), torch.empty_like(q)
+        rc = lib.alpx_prefill_causal(
+            q.data_ptr(), K.data_ptr(), V.data_ptr(), out.data_ptr(), ws.data_ptr(), nbytes, tq,
+            total, hq, hkv, d, d, hkv * d, hkv * d, prefix, 0, 0, scale, Lib.F32, Lib.F32,
+            Lib.stream_handle(torch, gpu))
+        torch.cuda.synchronize()
+        assert rc == Lib.OK
+        return out
+
+    assert torch.equal(call(want), fresh)
+    Lib.timing_enable(True)
+    try:
+        short = call(least)
+        launches = [Lib.timing_read(k)[1] for k in (Lib.T_PREFILL, Lib.T_AUX)]
+    finally:
+        Lib.timing_enable(False)
+    assert launches == [1, 0 if least_runs == "f32" else 1]
+    # other pieces: the same float32 products and sums in another order
+    assert (short - fresh).abs().max().item() <= 2e-5
+    ref = A.attention_batch(*(x.cpu().numpy() for x in (q, K, V)), prefix + np.arange(tq),
+                            hq // hkv, scale)
+    assert np.abs(fresh.cpu().numpy() - ref).max() <= TOL["f32"]
+
+
 def test_prefill_append_range_error_leaves_cache(gpu):
     import torch
     P = _mod("_ops")
