@@ -442,7 +442,8 @@ def prefill(q, key, value, *, pos0, scale=None, window=0, kv_start=0, kv_tokens=
         args = (None if workspace is None else workspace.data_ptr(), size, q_tokens,
                 int(kv_tokens), q_heads, kv_heads, key_dim, value_dim, int(k_pos_stride),
                 int(v_pos_stride), int(pos0), int(window), int(kv_start), float(scale),
-                _lib.dtype_code(torch, q.dtype), _lib.dtype_code(torch, out.dtype), _lib.stream_handle(torch, q.device))
+                _lib.dtype_code(torch, q.dtype), _lib.dtype_code(torch, out.dtype),
+                _lib.stream_handle(torch, q.device))
         if gate is None:
             return L.alpx_prefill_causal(q.data_ptr(), key.data_ptr(), value.data_ptr(),
                                          out.data_ptr(), *args)
@@ -829,7 +830,8 @@ def attention_layer_prefill(query_gate, key, value, q_norm, k_norm, key_cache, v
     rc = call(query, own(split))
     if rc == _lib.EINVAL:  # the split-K prefill (fp32, unaligned, >= 2 GiB) needs a workspace
         total = int(position) + tokens
-        nbytes = (_f32_prefill_bytes(tokens, total, q_heads, kv_heads, dim, dim, int(position), 0, 0)
+        nbytes = (_f32_prefill_bytes(tokens, total, q_heads, kv_heads, dim, dim, int(position), 0,
+                                     0)
                   if key_cache.dtype == torch.float32
                   else L.alpx_prefill_workspace_bytes(tokens, q_heads, kv_heads, dim, total))
         if nbytes == 0:

@@ -107,6 +107,12 @@ extern "C" size_t alpx_prefill_workspace_bytes(int q_tokens, int q_heads, int kv
 
 namespace {
 
+// The window, or 0 where it reaches back past row 0 for every token (it hides
+// nothing then): the kernels form its positions in 32 bits.
+int live_window(int window, int64_t rel0, int q_tokens) {
+  return (int64_t)window >= rel0 + q_tokens ? 0 : window;
+}
+
 // Key tiles (of `rows` rows) that column tile ct walks: tile_keys on the host.
 int host_tile_keys(int q_tokens, int kv_tokens, int group, int rel0, int window, int cols_per_block,
                    int rows, int ct) {
@@ -342,6 +348,7 @@ int prefill_impl(const void* q, const void* key, const void* value, const void* 
   if (key_dim > 256 || value_dim > 256)
     return fail(ALPX_EUNSUPPORTED, "alpx_prefill_causal: head dims above 256 are not supported");
 
+  window = live_window(window, q_pos0 - kv_start, q_tokens);
   hipStream_t s = (hipStream_t)stream;
   const int group = q_heads / kv_heads;
   const size_t es = dtype_size(dtype);
@@ -535,7 +542,9 @@ extern "C" size_t alpx_prefill_split_bytes(int q_tokens, int kv_tokens, int q_he
       q_heads % kv_heads != 0 || (head_dim != 64 && head_dim != 128 && head_dim != 256) ||
       window < 0 || rel0 >= ((int64_t)1 << 30) || rel0 <= -((int64_t)1 << 30))
     return 0;
-  return plan_split_prefill(q_tokens, kv_tokens, q_heads, kv_heads, head_dim, rel0, window).bytes;
+  return plan_split_prefill(q_tokens, kv_tokens, q_heads, kv_heads, head_dim, rel0,
+                            live_window(window, rel0, q_tokens))
+      .bytes;
 }
 
 extern "C" size_t alpx_prefill_f32_workspace_bytes(int q_tokens, int kv_tokens, int q_heads,
@@ -550,7 +559,7 @@ extern "C" size_t alpx_prefill_f32_workspace_bytes(int q_tokens, int kv_tokens, 
       window >= 0 && rel0 < ((int64_t)1 << 30) && rel0 > -((int64_t)1 << 30) &&
       (int64_t)q_tokens * (q_heads / kv_heads) < ((int64_t)1 << 30))
     p = plan_split_f32(q_tokens, kv_tokens, kv_heads, q_heads / kv_heads, key_dim, (int)rel0,
-                       window, SIZE_MAX);
+                       live_window(window, rel0, q_tokens), SIZE_MAX);
   if (pieces != nullptr) *pieces = p.splits;
   return std::max(need, p.bytes);
 }

@@ -337,6 +337,23 @@ def test_prefill_f32_plan_follows_the_call_not_the_workspace(gpu, monkeypatch, t
     assert np.abs(fresh.cpu().numpy() - ref).max() <= TOL["f32"]
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("tq,pos0,kv_start,rows,window", [
+    (300, 45, 50, 295, 2**31 - 1), (300, 45, 50, 295, 2**31 - 4), (90, 700, 0, 790, 2**31 - 1),
+    (130, 400, 100, 430, 430), (20, 0, 50, 40, 2**31 - 1)])
+def test_prefill_window_that_hides_nothing(gpu, dtype, tq, pos0, kv_start, rows, window):
+    """A window that reaches back past the first cache row for every token,
+    up to the largest one, gives the bits of no window, also where the first
+    tokens come before that row."""
+    import torch
+    P = _mod("_ops")
+    gen = torch.Generator(device=gpu).manual_seed(tq)
+    r = lambda *s: torch.randn(*s, generator=gen, device=gpu).to(_tdtype(torch, dtype))  # noqa: E731
+    q, K, V = r(tq, 8, 64), r(rows, 8, 64), r(rows, 8, 64)
+    a, b = (P.prefill(q, K, V, pos0=pos0, kv_start=kv_start, window=w) for w in (window, 0))
+    assert torch.equal(a, b)
+
+
 def test_prefill_append_range_error_leaves_cache(gpu):
     import torch
     P = _mod("_ops")
