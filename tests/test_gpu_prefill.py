@@ -122,7 +122,7 @@ def test_prefill_append_equals_append_then_prefill(gpu, override, kernel, dtype,
     tile), no prefix, a group size that does not divide a block's columns
     (tokens whose columns span two blocks), head_dim 256 and windows."""
     import torch
-    override("prefill_kernel", kernel)  # fp32 takes the split-K path either way
+    override("prefill_kernel", kernel)  # fp16 / bf16 only: fp32 has one kernel
     P = _mod("_ops")
     rng = np.random.default_rng(tq * 13 + prefix + d + window)
     cap = prefix + tq + 9
@@ -209,36 +209,69 @@ def test_prefill_split_matches_unsplit_and_oracle(gpu, ops, override, dtype, tq,
     assert np.abs(outs[0].cpu().numpy() - ref).max() <= TOL[dtype]
 
 
-@pytest.mark.parametrize("tq,prefix,hq,hkv,d,window,pos_off,gated,out", [
-    (70, 0, 8, 2, 64, 0, 0, False, "f32"), (130, 43, 6, 2, 128, 50, 0, True, "f32"),
-    (67, 0, 16, 2, 256, 0, 0, False, "f16"), (1100, 0, 3, 1, 64, 0, 0, False, "f32"),
-    (20, 1500, 8, 2, 64, 0, 0, False, "f32"), (33, 701, 12, 4, 128, 600, 0, True, "bf16"),
-    (50, 2001, 16, 2, 256, 0, 0, True, "f32"), (300, 0, 8, 8, 64, 0, -5, False, "f32"),
-    (363, 285, 2, 2, 256, 332, 0, False, "f32"), (500, 100, 4, 2, 64, 200, 0, False, "f32"),
-    (1, 4096, 4, 1, 128, 0, 0, False, "f32"), (9, 31, 40, 2, 128, 0, 0, False, "f32")])
+def _f32_plan(tq, total, hq, hkv, d, pos0, window=0, kv_start=0):
+    """How the library runs a float32 chunk: "decode" (the decode machinery),
+    "whole" key ranges or "pieces" of them."""
+    import ctypes
+    n = ctypes.c_int()
+    assert _mod("_lib").lib().alpx_prefill_f32_workspace_bytes(
+        tq, total, hq, hkv, d, d, pos0, window, kv_start, ctypes.byref(n)) > 0
+    return "decode" if n.value < 0 else "pieces" if n.value else "whole"
+
+
+@pytest.mark.parametrize("tq,prefix,hq,hkv,d,window,pos_off,gated,out,plan", [
+    (1000, 0, 32, 8, 64, 0, 0, False, "f32", "whole"),
+    (67, 31, 40, 8, 64, 0, 0, True, "bf16", "whole"),
+    (700, 0, 48, 8, 128, 0, 0, True, "f32", "whole"),
+    (203, 43, 24, 8, 128, 50, 0, False, "f16", "whole"),
+    (203, 57, 24, 8, 256, 64, 0, True, "f32", "whole"),
+    (300, 0, 64, 16, 64, 200, -5, False, "f32", "whole"),
+    (1100, 0, 3, 1, 64, 0, 0, False, "f32", "pieces"),
+    (65, 43, 8, 8, 64, 50, 0, True, "f16", "pieces"),
+    (33, 701, 12, 4, 128, 600, 0, True, "bf16", "pieces"),
+    (65, 43, 8, 8, 128, 50, 0, False, "f32", "pieces"),
+    (50, 2001, 16, 2, 256, 0, 0, True, "f32", "pieces"),
+    (300, 0, 8, 8, 64, 0, -5, False, "f32", "pieces"),
+    (363, 285, 2, 2, 256, 332, 0, False, "f32", "pieces"),
+    (500, 100, 4, 2, 64, 200, 0, False, "f32", "pieces"),
+    (70, 0, 8, 2, 64, 0, 0, False, "f32", "decode"),
+    (130, 43, 6, 2, 128, 50, 0, True, "f32", "decode"),
+    (67, 0, 16, 2, 256, 0, 0, False, "f16", "decode"),
+    (20, 1500, 8, 2, 64, 0, 0, False, "f32", "decode"),
+    (1, 4096, 4, 1, 128, 0, 0, False, "f32", "decode"),
+    (9, 31, 40, 2, 128, 0, 0, False, "f32", "decode")])
 def test_prefill_f32_matches_oracle_and_decode_machinery(gpu, override, tq, prefix, hq, hkv, d,
-                                                         window, pos_off, gated, out):
+                                                         window, pos_off, gated, out, plan):
     """float32 chunks: whole key ranges, pieces of them merged by a second
-    launch, and the few tokens left to the decode machinery; key counts that
-    are no multiple of a tile, columns that do not fill a block, groups that
-    do not divide it, windows, rows that see no key, the gate, 16-bit
-    outputs.  Against the oracle, and against the decode machinery (the same
-    float32 products in another order: 2e-5, ten times what was seen)."""
+    launch, and the few tokens left to the decode machinery (each row names
+    which, and the launches it made are counted); key counts that are no
+    multiple of a tile, columns that do not fill a block, groups that do not
+    divide it, windows, rows that see no key, the gate, 16-bit outputs.
+    Against the oracle, and against the decode machinery (the same float32
+    products in another order: 2e-5, ten times what was seen)."""
     import torch
-    P = _mod("_ops")
+    P, Lib = _mod("_ops"), _mod("_lib")
     total = prefix + tq
     rng = np.random.default_rng(tq + prefix + d)
     r = lambda *s: rng.standard_normal(s).astype(np.float32)  # noqa: E731
     q, K, V, gate = r(tq, hq, d), r(total, hkv, d), r(total, hkv, d), r(tq, hq, d)
     pos0 = prefix if pos_off == 0 else 50 + pos_off
     kv_start = 0 if pos_off == 0 else 50
+    assert _f32_plan(tq, total, hq, hkv, d, pos0, window, kv_start) == plan
     outs = []
     for generic in (0, 1):
         override("prefill_generic", generic)
-        outs.append(P.prefill(_dev(torch, q, "f32", gpu), _dev(torch, K, "f32", gpu),
-                              _dev(torch, V, "f32", gpu), pos0=pos0, kv_start=kv_start,
-                              window=window, out_dtype=_tdtype(torch, out),
-                              gate=_dev(torch, gate, "f32", gpu) if gated else None).float())
+        Lib.timing_enable(True)
+        try:
+            outs.append(P.prefill(_dev(torch, q, "f32", gpu), _dev(torch, K, "f32", gpu),
+                                  _dev(torch, V, "f32", gpu), pos0=pos0, kv_start=kv_start,
+                                  window=window, out_dtype=_tdtype(torch, out),
+                                  gate=_dev(torch, gate, "f32", gpu) if gated else None).float())
+            torch.cuda.synchronize()
+            combines = Lib.timing_read(Lib.T_AUX)[1]  # the decode machinery's second launch
+        finally:
+            Lib.timing_enable(False)
+        assert combines == (1 if generic or plan == "decode" else 0)
     ref = A.attention_batch(q, K, V, pos0 + np.arange(tq), hq // hkv, 1.0 / np.sqrt(d),
                             window=window, kv_start=kv_start)
     if gated:
@@ -263,6 +296,7 @@ def test_prefill_f32_unseen_rows_never_reach_a_row(gpu, tq, prefix, hq, hkv, d, 
     import torch
     P = _mod("_ops")
     total, slack = prefix + tq, 37
+    assert _f32_plan(tq, total + slack, hq, hkv, d, prefix, window) != "decode"
     rng = np.random.default_rng(tq + d)
     r = lambda *s: torch.from_numpy(rng.standard_normal(s).astype(np.float32)).to(gpu)  # noqa: E731
     q, K, V = r(tq, hq, d), r(total + slack, hkv, d), r(total + slack, hkv, d)
