@@ -516,10 +516,11 @@ __device__ __forceinline__ void split_body(const DecodeArgs& a, const SplitProlo
   // One walk over the wave's rows.  `lane` is a parameter, and opaque for the
   // second walk, so that the two share no addresses: held for both, they
   // pushed the first walk's into other registers.  At head_dim 256, where
-  // the loop has no register to spare, the scheduler then issued a tile's
-  // loads in another order than the loop stages them, which exposed them all
-  // (64 sequences of 1024 rows, 16/2 heads: 27.7 -> 35.5 us): the loads are
-  // kept in order there, two of each at a time (27.9; one 29.1).
+  // the loop has no register to spare, the scheduler may issue a tile's loads
+  // in another order than the loop stages them, which exposes them all: they
+  // are kept in order there, two of each at a time (out of order / in order /
+  // one of each at a time: one launch, 64 sequences of 1024 rows, 16/2 heads
+  // 35.5 / 27.9 / 29.1 us; split, layer step of 4 x 32768 rows 57.5 / 55.4).
   auto walk = [&](auto again, const int lane) __attribute__((always_inline)) {
     [[maybe_unused]] constexpr bool kAgain = decltype(again)::value;
     const int hl = lane & 15, quad = lane >> 4;
@@ -552,7 +553,7 @@ __device__ __forceinline__ void split_body(const DecodeArgs& a, const SplitProlo
         kr[it] = __builtin_bit_cast(V8, __builtin_amdgcn_raw_buffer_load_b128(kres, koff + it * kstep, 0, 0));
         vr[it] = __builtin_bit_cast(
             V8, __builtin_amdgcn_raw_buffer_load_b128(vres, voff + it * vstep, 0, kAuxNontemporal));
-        if (TWO && D == 256 && it % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+        if (D == 256 && it % 2 == 1) __builtin_amdgcn_sched_barrier(0);
       }
     };
 
