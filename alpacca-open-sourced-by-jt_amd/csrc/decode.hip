@@ -100,9 +100,9 @@ __device__ __forceinline__ int seq_lo(const DecodeArgs& a, int b, int hi) {
 // longest sequence.  Since sum_b ceil(len_b / C) <= total / C + batch <=
 // items_target + batch, the grid (items_max = items_target + batch) holds
 // every item; blocks past the last item exit.  Up to one_rows rows in all C
-// is cut for items_one blocks instead, so that the items run in one round.  The functions below are
-// wave-collective (every lane of the calling wave active) and every wave
-// that calls them gets the same result.
+// is cut for items_one blocks instead, so that the items run in one round.
+// The functions below are wave-collective (every lane of the calling wave
+// active) and every wave that calls them gets the same result.
 
 __device__ __forceinline__ int64_t wave_sum(int64_t x) {
 #pragma unroll

@@ -64,10 +64,7 @@ prefill_split(PrefillArgs a) {
       grp == 0 ? nullptr : a.part_st + slot * kCols);
 }
 
-// Merges the pieces of prefill_split: one block per (kv head, column tile,
-// 16 columns), the O fragments of the 16 columns shared out over its four
-// waves.  Each piece weighs 2^(mc - M), M the largest offset among the
-// column's pieces that saw a key; the gate is applied before the rounding.
+// sigmoid(g) as the kernels that the pieces stand in for form it.
 template <typename T>
 __device__ __forceinline__ float gate_factor(T g) {
   if constexpr (sizeof(T) == 4)
@@ -76,6 +73,11 @@ __device__ __forceinline__ float gate_factor(T g) {
     return fast_sigmoid(to_f32(g));
 }
 
+// Merges the pieces of prefill_split or prefill_f32: one block per (kv head,
+// column tile, 16 columns), the O fragments of the 16 columns shared out over
+// its four waves.  Each piece weighs 2^(mc - M), M the largest offset among
+// the column's pieces that saw a key; the gate is applied before the
+// rounding.
 template <typename T, typename TO, int D, int BK, int NQB>
 __global__ void __launch_bounds__(256)
 prefill_combine(PrefillArgs a) {

@@ -208,7 +208,9 @@ size_t alpx_decode_workspace_bytes(int batch, int q_heads, int kv_heads, int val
  * workspace must hold alpx_decode_workspace_bytes(batch, q_heads,
  * kv_heads, value_dim, length) bytes; it is scratch (no initial contents
  * needed).  Calls sharing a workspace must be ordered on one stream.  One
- * call is two kernel launches: the split pass and the combine pass.
+ * call is two kernel launches, the split pass and the combine pass, or one
+ * that leaves the workspace alone (short caches, and batches that fill the
+ * device with a block per sequence and kv head).
  */
 int alpx_decode_gqa(const void* q, const void* key_cache, const void* value_cache,
                     const int32_t* seq_lens, int length, const void* gate, void* out,
@@ -501,10 +503,11 @@ int alpx_attention_prologue(const void* query_gate, const void* key, const void*
 /* One decode token of the Qwen3.5 full-attention layer after its
  * projections (qwen35_runtime.py:597-665 for one token per sequence:
  * alpx_attention_prologue followed by alpx_decode_gqa with the sigmoid
- * gate), in two launches.  Sequence b's token sits at cache row pos_b =
- * positions[b] (device int32) or, with positions null, `position`; with
- * positions, `position` bounds them (a pos_b outside [0, position] writes
- * no cache row and attends rows 0 .. min(pos_b, position)).  The split-K
+ * gate), in the decode's launches (two, or one).  Sequence b's token sits at
+ * cache row pos_b = positions[b] (device int32) or, with positions null,
+ * `position`; with positions, `position` bounds them (a pos_b outside [0,
+ * position] writes no cache row and attends rows 0 .. min(pos_b, position)).
+ * The split-K
  * launch forms each block's query heads from query_gate [B, Hq, 2D]
  * (RMSNorm with q_norm, IMROPE at the text lanes (pos_b, pos_b, pos_b, 0))
  * and, in the blocks whose chunk holds row pos_b, the key row from key
@@ -602,7 +605,7 @@ int alpx_attention_prologue_chunk(const void* query_gate, const void* key, const
  * token-sequential Qwen35Model._attention calls of a prefill
  * (qwen35_runtime.py:597-665, prefill_state qwen35_runtime.py:777-810).
  * value_dim must equal head_dim (the gate has head_dim values per head);
- * workspace as alpx_prefill_causal (only its fallback path uses it).
+ * workspace as alpx_prefill_causal.
  *
  * query_out may be null: the prefill then forms the query rows itself from
  * query_gate (the prologue's RMSNorm and IMROPE in its query load, same
